@@ -178,11 +178,41 @@ int small_tile_rows(int N, int M) {
     return 2 * (int64_t)((N + 63) / 64) * ((M + 63) / 64) <= 3 * cus ? 32 : 64;
 }
 
+// The K-sliced mid-batch kernel's tile shape where it is estimated to beat the tiled GEMMs,
+// else -1.  Their time is a fixed part per 128-value stage plus one per workgroup (fitted to
+// K=4096 and 11008, N=2048..14336, 48..2048 tokens; 32-row tiles: 0.36 + 0.00076 us per
+// workgroup; 64: 0.31 + 0.00158; 128 x 128: 3.03 us per round of two workgroups per CU).
+// Measured, tiled against K-sliced (us): N=4096, K=4096: 48 tokens 21.6 / 8.4, 100: 22.3 /
+// 11.8, 512: 37.4 / 31.1, 2048: 105-110 / 112 (stays tiled); K=11008: 48: 52 / 18, 1024:
+// 157-167 / 140; N=14336, K=4096: 100: 37.6 / 31, 512: 105-117 / 98, 1024: 197 / 197.
+int kslice_shape(int K, int N, int M) {
+    if (M > 65535) return -1;
+    const double stages = K / kQSuper, cus = device_cus();
+    double tiled;
+    if (const int tr = small_tile_rows(N, M); tr != 0) {
+        const double wgs = (double)((N + tr - 1) / tr) * ((M + 63) / 64);
+        tiled = 4.0 + stages * (tr == 32 ? 0.36 + 0.00076 * wgs : 0.31 + 0.00158 * wgs);
+    } else {
+        const double tiles = (double)((N + 127) / 128) * ((M + 127) / 128);
+        tiled = 5.0 + stages * 3.03 * (tiles / (2.0 * cus) + 0.1);
+    }
+    double sliced;
+    const int shape = kslice_pick(K, N, M, &sliced);
+    return sliced < 0.97 * tiled ? shape : -1;
+}
+
+int run_kslice(const void *w, const void *xq, float *y, int K, int N, int M, bool split, int shape, hipStream_t s) {
+    const hipError_t e = launch_gemm_kslice(w, xq, y, K, N, M, split, shape, s);
+    return e == hipSuccess ? JJO_OK : hip_fail(e, "gemm_kslice launch");
+}
+
 int run_mm(const void *w, const void *xq, float *y, int K, int N, int M, int algo, hipStream_t s) {
     if (algo == JJO_ALGO_AUTO) {
         const bool gemv_ok = M <= kGemvMaxBatch && K <= kGemvMaxK && (int64_t)M * (K / 64) * 80 <= 150 * 1024;
         // The GEMV wins up to batch 4 on rows of one K-slice (K <= 4096); with more
         // slices its per-token cost grows and the skinny kernel wins from batch 3.
+        // Above batch 16 the K-sliced GEMM replaces both skinny kernels (24 tokens, N=14336,
+        // K=4096: 25.1 -> 16.2 us; N=4096, K=11008: 27.6 -> 18.5 us).
         // At K <= 4096 the LDS-resident skinny kernel is 4-30% faster than the
         // per-wave one from batch 5 (N=14336: 11.2-11.6 against 12.0-14.0 us; N=11008:
         // 9.0-9.4 against 11.5-13.4 us); at larger K the per-wave kernel is faster.
@@ -190,10 +220,14 @@ int run_mm(const void *w, const void *xq, float *y, int K, int N, int M, int alg
             algo = JJO_ALGO_GEMV;
         else if (K <= 4096 && M >= 5 && gemm_skinny_persist_supported(w, xq, K, M))
             algo = JJO_ALGO_SKINNY_LDS;
-        else if (gemm_skinny_supported(w, xq, K, M))
+        else if (M <= 16 && gemm_skinny_supported(w, xq, K, M))
             algo = JJO_ALGO_SKINNY;
         else if (gemv_ok)
             algo = JJO_ALGO_GEMV;
+        else if (const int shape = kslice_shape(K, N, M); shape >= 0)
+            return run_kslice(w, xq, y, K, N, M, false, shape, s);
+        else if (gemm_skinny_supported(w, xq, K, M))
+            algo = JJO_ALGO_SKINNY;
         else if (const int tr = small_tile_rows(N, M); tr != 0)
             algo = tr == 32 ? JJO_ALGO_MFMA32 : JJO_ALGO_MFMA64;
         else
@@ -423,8 +457,9 @@ int run_mm_split(const void *w, const void *xq, float *y, int K, int N, int M, h
     const bool gemv_ok = M <= kGemvMaxBatch && K <= kGemvMaxK && (int64_t)M * (K / kQK) * 48 <= 150 * 1024;
     // The block_q4_0 AUTO dispatch's choices, each kernel reading the split layout: the
     // GEMV up to batch 4 (one K slice) or 2, the LDS-resident skinny kernel for 5..16 at
-    // K <= 4096, the per-wave skinny kernel up to 32, then the small-tile GEMM while the
-    // 128 x 128 tiles would not fill the chip well, else the 128 x 128 GEMM.
+    // K <= 4096, the per-wave skinny kernel up to 16, then the K-sliced GEMM where it is
+    // faster than the tiled ones, the small-tile GEMM while the 128 x 128 tiles would not
+    // fill the chip well, else the 128 x 128 GEMM.
     hipError_t e;
     if (gemv_ok && M <= (K <= 4096 ? kGemvPreferredBatch : 2)) {
         e = launch_gemv_q4s(w, xq, y, K, N, M, s);
@@ -434,7 +469,7 @@ int run_mm_split(const void *w, const void *xq, float *y, int K, int N, int M, h
         e = launch_gemm_skinny_persist_layout(w, xq, y, K, N, M, true, s);
         return e == hipSuccess ? JJO_OK : hip_fail(e, "gemm_skinny_persist (split layout) launch");
     }
-    if (gemm_skinny_supported(w, xq, K, M)) {
+    if (M <= 16 && gemm_skinny_supported(w, xq, K, M)) {
         e = launch_gemm_skinny_layout(w, xq, y, K, N, M, true, s);
         return e == hipSuccess ? JJO_OK : hip_fail(e, "gemm_skinny (split layout) launch");
     }
@@ -442,7 +477,11 @@ int run_mm_split(const void *w, const void *xq, float *y, int K, int N, int M, h
         e = launch_gemv_q4s(w, xq, y, K, N, M, s);
         return e == hipSuccess ? JJO_OK : hip_fail(e, "gemv_q4s launch");
     }
-    // K=14336, N=4096, M=48 on the 128 x 128 split GEMM: 126 us (32 workgroups).
+    if (const int shape = kslice_shape(K, N, M); shape >= 0) return run_kslice(w, xq, y, K, N, M, true, shape, s);
+    if (gemm_skinny_supported(w, xq, K, M)) {
+        e = launch_gemm_skinny_layout(w, xq, y, K, N, M, true, s);
+        return e == hipSuccess ? JJO_OK : hip_fail(e, "gemm_skinny (split layout) launch");
+    }
     if (const int tr = small_tile_rows(N, M); tr != 0) {
         e = launch_gemm_mfma64(w, xq, y, K, N, M, s, tr, true);
         return e == hipSuccess ? JJO_OK : hip_fail(e, "gemm_mfma64 (split layout) launch");

@@ -1,0 +1,374 @@
+// Mid-batch GEMM (about 17 to 1000 tokens) of Q4_0 weights x Q8_1 activations on
+// gfx950 int8 matrix cores: the K range of an output tile is cut over the waves of
+// one workgroup.
+//
+// Math is the reference's per-block epilogue (src/cuda/mm_q4_0_q8_1.cu:71-93,
+// summed over K at :256-269):
+//     y[m][n] = sum_b d_w[n,b] * (sumi[n,m,b] * d_x[m,b] - 8 * s_x[m,b])
+// with the exact int32 block sums of v_mfma_i32_32x32x32_i8 read as fp32 through the
+// 1.5*2^23 accumulator bias (mfma_q4q8_tile.hpp), two fp32 FMAs per element and block,
+// and the s_x term on an f16 MFMA.
+//
+// What bounds it, and the design that follows
+//   * A batch of tens or hundreds of tokens has too few 64- or 128-row tiles for 256
+//     CUs: N=4096, K=11008, 48 tokens ran 128 workgroups of four waves, each wave
+//     walking all of K, at 52 us.  Here a workgroup is WK waves that each own a
+//     contiguous K slice of the SAME (32*RT rows) x (32*CT tokens) tile, so a small
+//     output still fills the chip with waves (18 us).  The slices' partial sums are
+//     added through LDS in slice order; no workspace, no atomics, no second launch, and
+//     the result does not depend on timing.
+//   * A wave shares nothing with the others inside the K loop, so there is no barrier in
+//     it.  A stage (128 of K: one Q8_1 superblock) moves to the wave's own LDS with LDS
+//     DMA (activations: 1 KB contiguous runs; weights: 64 nibble bytes or one 72-byte
+//     run per row), is read into registers, and the DMA of the next stage starts into
+//     the same bytes while this one is computed.  Direct loads of the MFMA operands
+//     (16 bytes every 144 for the activation) touch a cache line per lane pair and ran
+//     at half the speed (K=4096, N=14336, 64 tokens: 33 us against 22).
+//   * One buffer per wave, not a ring: deeper rings hid no more latency and cost
+//     residency (64 x 64 tiles, 256 tokens, N=14336, block_q4_0: 83 us with two weight
+//     slots, 59 with one).
+//   * The loop is bound by instruction issue: a wave issues a two-operand VALU
+//     instruction every 5.0 clocks and a three-operand one every 6.1, a SIMD every 2.5
+//     and 3.1 from two waves on, and MFMA time adds to it almost in full.  So what is
+//     minimised is instructions per 32x32 block: weights are expanded with one load of
+//     two blocks per lane pair and v_permlane32_swap (no duplicated work in the two lane
+//     halves), scales are widened to fp32 once per stage, d_x stays an fp32 register (a
+//     v_fma_mix would issue at two thirds of the rate), and the next block's MFMA is
+//     issued before the epilogue that the previous one feeds (sched_barrier: left alone,
+//     the scheduler sinks it behind that epilogue, 5-10% slower).
+//   * Tile shapes: kslice_pick() below.
+#include <hip/hip_fp16.h>
+
+#include "mfma_q4q8_tile.hpp"
+#include "q4q8_common.hpp"
+
+namespace jjo {
+namespace {
+
+typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
+
+// One wave's staging area: activations [32*CT][144], weights per row tile (split: 32 x 64
+// nibble bytes and 32 x 8 scale bytes; block_q4_0: 32 rows x 6 chunks of 12 bytes at a
+// 16-byte stride, the layout of a 12-byte LDS DMA), fp32 scales [RT][4][32].
+template <int RT, int CT, bool SPLIT>
+struct KsliceLds {
+    static constexpr int kXBytes = 32 * CT * kQ8BlockBytes;
+    static constexpr int kXRuns = (kXBytes + 1023) / 1024;  // the last may be half a run
+    static constexpr int kWTile = SPLIT ? 2048 + 256 : 3072;
+    static constexpr int kOffW = kXBytes;
+    static constexpr int kOffScale = kOffW + RT * kWTile;
+    static constexpr int kWave = kOffScale + RT * 512;
+};
+
+template <int RT, int CT, int WK, bool SPLIT, int WAVES_PER_SIMD>
+__global__ __launch_bounds__(64 * WK, WAVES_PER_SIMD) void gemm_kslice_kernel(
+    const uint8_t *__restrict__ w, const uint8_t *__restrict__ xq, float *__restrict__ y, int K, int N, int M,
+    int row_tiles, int tok_tiles) {
+    using L = KsliceLds<RT, CT, SPLIT>;
+    extern __shared__ __align__(16) uint8_t smem[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, hh = lane >> 5;
+
+    // Workgroups go round-robin over the 8 XCDs: the token tiles of a row tile follow each
+    // other on one XCD, so its weights come from HBM once.
+    int row_tile = blockIdx.x, tok_tile = 0;
+    if (tok_tiles > 1) {
+        const int slot = blockIdx.x >> 3;
+        row_tile = (slot / tok_tiles) * 8 + (blockIdx.x & 7);
+        tok_tile = slot % tok_tiles;
+        if (row_tile >= row_tiles) return;  // uniform over the workgroup
+    }
+    const int n0 = row_tile * 32 * RT, m0 = tok_tile * 32 * CT;
+    const int nb = K / kQK, nsb = K / kQSuper;
+
+    // ---- staging: rows past N and tokens past M re-read the last valid one ----
+    const uint8_t *wq = w + (size_t)n0 * nb * (SPLIT ? 16 : kQ4BlockBytes);
+    const uint8_t *wd = w + ((size_t)N * 16 + (size_t)n0 * 2) * nb;  // split: the scale plane
+    const uint8_t *xb = xq + (size_t)m0 * kQ8BlockBytes;
+    const size_t x_stride = (size_t)M * kQ8BlockBytes;
+    uint8_t *stage = smem + wave * L::kWave;
+    const uint32_t stage_lds = (uint32_t)(uintptr_t)stage;
+    float *wde = reinterpret_cast<float *>(stage + L::kOffScale);
+    const uint32_t xlim = min(32 * CT, M - m0) * kQ8BlockBytes - 16;
+    uint32_t woff[RT][3];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        const int last = N - 1 - n0;
+        if constexpr (SPLIT) {
+            // lane l: row l/4 of 16, block (l%4) ^ ((row/4)%4): the 16 rows that read one
+            // block then fall in 16 different 16-byte bank groups
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                woff[rt][i] = (uint32_t)min(32 * rt + 16 * i + (lane >> 2), last) * nb * 16 +
+                              16 * ((lane & 3) ^ ((lane >> 4) & 3));
+            woff[rt][2] = (uint32_t)min(32 * rt + l32, last) * nb * 2 + 4 * hh;
+        } else {
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                const int c = 64 * i + lane;
+                woff[rt][i] = (uint32_t)min(32 * rt + c / 6, last) * nb * kQ4BlockBytes + 12 * (c % 6);
+            }
+        }
+    }
+    // Inline asm: the compiler would order every later LDS access behind these; their
+    // completion is waited for at the top of a stage.
+    auto dma = [&](int s) {
+        const uint8_t *px = xb + (size_t)s * x_stride;
+#pragma unroll
+        for (int i = 0; i < L::kXRuns; ++i) {
+            const uint32_t m0v = __builtin_amdgcn_readfirstlane(stage_lds + i * 1024);
+            if ((i + 1) * 1024 <= L::kXBytes || lane < 32)
+                asm volatile("global_load_lds_dwordx4 %0, %1"
+                             :
+                             : "v"(min((uint32_t)(i * 1024 + lane * 16), xlim)), "s"(px), "{m0}"(m0v)
+                             : "memory");
+        }
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            const uint32_t dst = stage_lds + L::kOffW + rt * L::kWTile;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                const uint32_t m0v = __builtin_amdgcn_readfirstlane(dst + i * 1024);
+                if constexpr (!SPLIT)
+                    asm volatile("global_load_lds_dwordx3 %0, %1"
+                                 :
+                                 : "v"(woff[rt][i]), "s"(wq + (size_t)s * (4 * kQ4BlockBytes)), "{m0}"(m0v)
+                                 : "memory");
+                else if (i < 2)
+                    asm volatile("global_load_lds_dwordx4 %0, %1"
+                                 :
+                                 : "v"(woff[rt][i]), "s"(wq + (size_t)s * 64), "{m0}"(m0v)
+                                 : "memory");
+                else
+                    asm volatile("global_load_lds_dword %0, %1"
+                                 :
+                                 : "v"(woff[rt][i]), "s"(wd + (size_t)s * 8), "{m0}"(m0v)
+                                 : "memory");
+            }
+        }
+    };
+
+    i32x16 bias;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) bias[v] = (int32_t)kBiasBits;
+    asm volatile("" : "+v"(bias));
+    f32x16 acc[RT][CT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[rt][ct][v] = 0.0f;
+
+    // Order of a stage's four blocks: a lane holds blocks 2*hh and 2*hh+1 of its row, so the
+    // first half-wave swap completes blocks 0 and 2, the second blocks 1 and 3.
+    constexpr int kOrder[4] = {0, 2, 1, 3};
+    constexpr int kJobs = 4 * RT * CT;  // 32x32 blocks of a stage
+    const int s_beg = (int)((int64_t)wave * nsb / WK), s_end = (int)((int64_t)(wave + 1) * nsb / WK);
+    if (s_beg < s_end) dma(s_beg);
+    for (int s = s_beg; s < s_end; ++s) {
+        JJO_GEMM_VMCNT(0);  // stage s has landed
+        asm volatile("" ::: "memory");
+        uint32_t raw[RT][9];
+        i32x4 xv[CT][4];
+        u32x4 hdr[CT];
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            const uint8_t *p = stage + L::kOffW + rt * L::kWTile;
+            if constexpr (SPLIT) {
+                const int sw = (l32 >> 2) & 3;
+                const u32x4 a = *reinterpret_cast<const u32x4 *>(p + l32 * 64 + 16 * ((2 * hh) ^ sw));
+                const u32x4 b = *reinterpret_cast<const u32x4 *>(p + l32 * 64 + 16 * ((2 * hh + 1) ^ sw));
+#pragma unroll
+                for (int k = 0; k < 4; ++k) { raw[rt][k] = a[k]; raw[rt][4 + k] = b[k]; }
+                raw[rt][8] = *reinterpret_cast<const uint32_t *>(p + 2048 + lane * 4);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 3; ++i) {
+                    const u32x3 a = *reinterpret_cast<const u32x3 *>(p + (l32 * 6 + 3 * hh + i) * 16);
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) raw[rt][3 * i + k] = a[k];
+                }
+            }
+        }
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+            const uint8_t *p = stage + (32 * ct + l32) * kQ8BlockBytes;
+            hdr[ct] = *reinterpret_cast<const u32x4 *>(p);
+#pragma unroll
+            for (int b = 0; b < 4; ++b) xv[ct][b] = *reinterpret_cast<const i32x4 *>(p + 16 + 32 * b + 16 * hh);
+        }
+        asm volatile("" ::: "memory");
+        JJO_GEMM_LGKM0();  // stage s is in registers: its bytes may be overwritten
+        asm volatile("" ::: "memory");
+        if (s + 1 < s_end) dma(s + 1);
+
+        // ---- weights: nibbles -> int8 operands of the four blocks, scales/8 -> fp32 ----
+        uint32_t d16[RT];  // the lane's two fp16 scales: its K slots of the s_x MFMA
+        i32x4 aop[RT][4];
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            uint32_t q[2][4];
+            if constexpr (SPLIT) {
+                d16[rt] = raw[rt][8];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) { q[0][k] = raw[rt][k]; q[1][k] = raw[rt][4 + k]; }
+            } else {
+                d16[rt] = (raw[rt][0] & 0xffffu) | (raw[rt][4] & 0xffff0000u);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    q[0][k] = __builtin_amdgcn_alignbyte(raw[rt][k + 1], raw[rt][k], 2);
+                    q[1][k] = raw[rt][5 + k];
+                }
+            }
+            float *dst = wde + rt * 128 + 2 * hh * 32 + epi_perm(l32);
+            dst[0] = 0.125f * __half2float(__ushort_as_half((unsigned short)(d16[rt] & 0xffffu)));
+            dst[32] = 0.125f * __half2float(__ushort_as_half((unsigned short)(d16[rt] >> 16)));
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    // lanes 0-31 hold block i, lanes 32-63 block 2+i; after the swap the first
+                    // register is block i (low nibbles | high nibbles), the second block 2+i
+                    const auto r = __builtin_amdgcn_permlane32_swap(q[i][k] & 0x0f0f0f0fu,
+                                                                    (q[i][k] >> 4) & 0x0f0f0f0fu, false, false);
+                    aop[rt][i][k] = (int32_t)r[0];
+                    aop[rt][2 + i][k] = (int32_t)r[1];
+                }
+        }
+
+        // ---- 32x32 blocks: the MFMA of block j+1 runs under the epilogue of block j ----
+        i32x16 d[2];
+        float wv[16];
+        auto load_wv = [&](int g) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const f32x4 v = *reinterpret_cast<const f32x4 *>(wde + (g % RT) * 128 + kOrder[g / RT] * 32 + 16 * hh + 4 * i);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) wv[4 * i + k] = v[k];
+            }
+        };
+        load_wv(0);
+        d[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(aop[0][kOrder[0]], xv[0][kOrder[0]], bias, 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < kJobs; ++j) {
+            const int rt = (j / CT) % RT, ct = j % CT, b = kOrder[j / (RT * CT)];
+            if (j + 1 < kJobs) {
+                const int rn = ((j + 1) / CT) % RT, cn = (j + 1) % CT, bn = kOrder[(j + 1) / (RT * CT)];
+                d[(j + 1) & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(aop[rn][bn], xv[cn][bn], bias, 0, 0, 0);
+            }
+            if (ct == 0 && j > 0) load_wv(j / CT);
+            float dx = __half2float(__ushort_as_half((unsigned short)(hdr[ct][b] & 0xffffu)));
+            asm("" : "+v"(dx));  // keep it fp32: no v_fma_mix in the epilogue
+            __builtin_amdgcn_sched_barrier(0);
+            epilogue_f32(acc[rt][ct], d[j & 1], wv, dx, dx * -kBias);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // sum_b d_w * (-s_x) of the stage: lane half hh holds blocks 2*hh and 2*hh+1 in its
+        // first two K slots of both operands, zeros in the others.
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+            const uint32_t h0 = hh ? hdr[ct][2] : hdr[ct][0], h1 = hh ? hdr[ct][3] : hdr[ct][1];
+            const u32x2 sx = {((h0 >> 16) | (h1 & 0xffff0000u)) ^ 0x80008000u, 0u};
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                const u32x2 dw = {d16[rt], 0u};
+                acc[rt][ct] = __builtin_amdgcn_mfma_f32_32x32x8f16(
+                    __builtin_bit_cast(f16x4, dw), __builtin_bit_cast(f16x4, sx), acc[rt][ct], 0, 0, 0);
+            }
+        }
+    }
+
+    // ---- add the K slices in slice order, y[m][n] = 8 * sum ----
+    __syncthreads();  // every wave is done with its staging area
+    f32x4 *red = reinterpret_cast<f32x4 *>(smem);
+    constexpr int kItems = RT * CT * 256;
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                red[wave * kItems + (rt * CT + ct) * 256 + q * 64 + lane] =
+                    f32x4{acc[rt][ct][4 * q], acc[rt][ct][4 * q + 1], acc[rt][ct][4 * q + 2], acc[rt][ct][4 * q + 3]};
+    __syncthreads();
+    // Eight consecutive threads take the 32 rows of one token: 128 contiguous bytes of y.
+    for (int it = tid; it < kItems; it += 64 * WK) {
+        const int qh = it & 7, tok = (it >> 3) & 31, tile = it >> 8;
+        const int src = tile * 256 + (qh >> 1) * 64 + tok + 32 * (qh & 1);
+        f32x4 v = red[src];
+#pragma unroll
+        for (int i = 1; i < WK; ++i) v += red[i * kItems + src];
+        v *= 8.0f;
+        const int m = m0 + 32 * (tile % CT) + tok, n = n0 + 32 * (tile / CT) + 4 * qh;
+        if (m >= M) continue;
+        float *yr = y + (size_t)m * N + n;
+        if (n + 3 < N && (N & 3) == 0) {
+            *reinterpret_cast<f32x4 *>(yr) = v;
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (n + k < N) yr[k] = v[k];
+        }
+    }
+}
+
+template <int RT, int CT, int WK, int WAVES_PER_SIMD>
+hipError_t launch(const void *w, const void *xq, float *y, int K, int N, int M, bool split, hipStream_t stream) {
+    auto kern = split ? gemm_kslice_kernel<RT, CT, WK, true, WAVES_PER_SIMD>
+                      : gemm_kslice_kernel<RT, CT, WK, false, WAVES_PER_SIMD>;
+    const size_t stage = WK * (size_t)(split ? KsliceLds<RT, CT, true>::kWave : KsliceLds<RT, CT, false>::kWave);
+    const size_t red = (size_t)WK * RT * CT * 4096, lds = stage > red ? stage : red;
+    hipError_t e = ensure_dynamic_lds((const void *)kern, lds);
+    if (e != hipSuccess) return e;
+    const int64_t rows = ((int64_t)N + 32 * RT - 1) / (32 * RT), toks = ((int64_t)M + 32 * CT - 1) / (32 * CT);
+    const int64_t grid = toks == 1 ? rows : (rows + 7) / 8 * 8 * toks;
+    if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * WK), lds, stream, (const uint8_t *)w,
+                       (const uint8_t *)xq, y, K, N, M, (int)rows, (int)toks);
+    return hipGetLastError();
+}
+
+// The tile shapes, with the time one CU takes for a 128-value stage of one workgroup's
+// tile (us, measured at K=4096, 11008 and 14336 with N=2048..14336 and 24..1024 tokens),
+// with its slots full and with a single workgroup on the CU.
+struct Shape {
+    int rt, ct;
+    double us, us_alone;
+};
+constexpr Shape kShapes[] = {
+    {1, 1, 0.14, 0.14},  // 8 waves, two workgroups per CU
+    {1, 2, 0.25, 0.25},  // 8 waves, one workgroup per CU
+    {2, 2, 0.46, 0.46},  // 8 waves, one workgroup per CU
+    {2, 2, 0.42, 0.51},  // 4 waves, two workgroups per CU
+};
+
+}  // namespace
+
+int kslice_pick(int K, int N, int M, double *us) {
+    const int64_t cus = device_cu_count();
+    int best = 0;
+    for (int i = 0; i < (int)(sizeof(kShapes) / sizeof(kShapes[0])); ++i) {
+        const Shape &s = kShapes[i];
+        const int64_t g = (((int64_t)N + 32 * s.rt - 1) / (32 * s.rt)) * (((int64_t)M + 32 * s.ct - 1) / (32 * s.ct));
+        const double t = 3.5 + (K / kQSuper) * (double)((g + cus - 1) / cus) * (g > cus ? s.us : s.us_alone);
+        if (i == 0 || t < *us) {
+            best = i;
+            *us = t;
+        }
+    }
+    return best;
+}
+
+hipError_t launch_gemm_kslice(const void *w, const void *xq, float *y, int K, int N, int M, bool split, int shape,
+                              hipStream_t stream) {
+    switch (shape) {
+        case 0: return launch<1, 1, 8, 4>(w, xq, y, K, N, M, split, stream);
+        case 1: return launch<1, 2, 8, 2>(w, xq, y, K, N, M, split, stream);
+        case 2: return launch<2, 2, 8, 2>(w, xq, y, K, N, M, split, stream);
+        default: return launch<2, 2, 4, 2>(w, xq, y, K, N, M, split, stream);
+    }
+}
+
+}  // namespace jjo

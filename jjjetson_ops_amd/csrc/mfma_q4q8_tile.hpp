@@ -35,6 +35,8 @@ constexpr float kBias = 12582912.0f;
 // s_waitcnt with only vmcnt constrained (gfx9 encoding: vmcnt[3:0] + [15:14],
 // expcnt[6:4] = 7, lgkmcnt[11:8] = 15).
 #define JJO_GEMM_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n)&15) | (((n) >> 4) << 14) | (7 << 4) | (15 << 8))
+// s_waitcnt lgkmcnt(0), vmcnt and expcnt unconstrained.
+#define JJO_GEMM_LGKM0() __builtin_amdgcn_s_waitcnt(0xC07F)
 
 // Position of tile-local row r (0..31) in the epilogue scale layout: the 16 rows
 // a lane half owns in the 32x32 MFMA output (rows 8q + 4h + i) become contiguous.

@@ -89,6 +89,12 @@ hipError_t launch_gemm_skinny_persist_layout(const void *w, const void *xq, floa
 // split: the weights are in the split layout (16-byte aligned).
 hipError_t launch_gemm_mfma64(const void *w, const void *xq, float *y, int K, int N, int M,
                               hipStream_t stream, int tile_rows, bool split = false);
+// Mid-batch GEMM, K cut over the waves of a workgroup (either layout; block_q4_0 4-byte,
+// split 16-byte aligned weights, any K % 128 == 0).  kslice_pick returns the tile shape
+// for a problem and its estimated time in microseconds.
+int kslice_pick(int K, int N, int M, double *us);
+hipError_t launch_gemm_kslice(const void *w, const void *xq, float *y, int K, int N, int M, bool split, int shape,
+                              hipStream_t stream);
 hipError_t launch_gemm_mfma(const void *w, const void *xq, float *y, int K, int N, int M,
                             hipStream_t stream);
 hipError_t launch_gemm_mfma_grouped(const void *w, const void *xq, const int32_t *expert_offsets,
