@@ -570,6 +570,36 @@ int mean_routes(int n_routes, int n_experts) {
     const int active = n_experts < n_routes ? n_experts : n_routes;
     return (n_routes + active - 1) / active;
 }
+// 32-route column tiles of the K-sliced grouped GEMM (one or two per workgroup), or 0 for
+// the 128-route tiles.  A 128-route tile with a handful of routes stages 128 weight rows for
+// one 32-column strip and is bound by that latency; the K-sliced form reads an expert's
+// weights with four waves per 64 rows.  FFN, us, 128-route tiles -> one / two column tiles
+// (block_q4_0): E=64 top-8 H=2048 I=1408, mean 2: 138 -> 124 / 132, 12.5: 158 -> 137 / 144,
+// 32: 210 -> 189 / 188, 64: 283 -> 293 / 279; E=8 top-2 H=4096 I=14336, mean 8: 292 -> 229
+// / 243, 25: 323 -> 248 / 262, 32: 475 -> 375 / 313, 64: 554 -> 542 / 488, 128: 798 -> 928 /
+// 804.  The mean hides the skew of a random router: from about 24 on, most launches hold
+// an expert above 32 routes, whose weights one column tile reads twice.
+int grouped_kslice_cols(int n_routes, int n_experts) {
+    const int mean = mean_routes(n_routes, n_experts);
+    return mean <= 24 ? 1 : mean <= 80 ? 2 : 0;
+}
+
+hipError_t run_grouped(const void *w, const void *w2, int n_split, const void *xq, const int32_t *offsets,
+                       int n_experts, const int32_t *route_dst, float *y, int K, int N, int n_routes, bool split,
+                       hipStream_t s) {
+    if (const int cols = grouped_kslice_cols(n_routes, n_experts); cols > 0)
+        return launch_gemm_kslice_grouped(w, w2, xq, y, nullptr, K, N, n_routes, n_split, offsets, n_experts,
+                                          route_dst, split, cols, s);
+    return launch_gemm_mfma_grouped(w, xq, offsets, n_experts, route_dst, y, K, N, n_routes, s, w2, n_split, split);
+}
+
+hipError_t run_gate_up_swiglu(const void *w_gate, const void *w_up, const void *xq, const int32_t *offsets,
+                              int n_experts, void *mid_q8_1, int K, int I, int n_routes, bool split, hipStream_t s) {
+    if (const int cols = grouped_kslice_cols(n_routes, n_experts); cols > 0)
+        return launch_gemm_kslice_grouped(w_gate, w_up, xq, nullptr, mid_q8_1, K, 2 * I, n_routes, I, offsets,
+                                          n_experts, nullptr, split, cols, s);
+    return launch_gemm_gate_up_swiglu_q8_1(w_gate, w_up, xq, offsets, n_experts, mid_q8_1, K, I, n_routes, s, split);
+}
 }  // namespace
 
 extern "C" {
@@ -589,8 +619,8 @@ int mat_mul_q4_0_q8_1_grouped_device(const void *d_w_q4_0, const void *d_x_q8_1,
                        ? launch_gemv_routed(d_w_q4_0, nullptr, d_x_q8_1, d_expert_offsets, n_experts, n_routes,
                                             mean_routes(n_routes, n_experts), d_y, nrows_out, ncols_k, nrows_out,
                                             false, (hipStream_t)stream, d_route_dst)
-                       : launch_gemm_mfma_grouped(d_w_q4_0, d_x_q8_1, d_expert_offsets, n_experts, d_route_dst,
-                                                  d_y, ncols_k, nrows_out, n_routes, (hipStream_t)stream);
+                       : run_grouped(d_w_q4_0, nullptr, 0, d_x_q8_1, d_expert_offsets, n_experts, d_route_dst, d_y,
+                                     ncols_k, nrows_out, n_routes, false, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "grouped gemm launch");
     return JJO_OK;
 }
@@ -610,9 +640,8 @@ int mat_mul_q4_0s_q8_1_grouped_device(const void *d_w_split, const void *d_x_q8_
                        ? launch_gemv_routed(d_w_split, nullptr, d_x_q8_1, d_expert_offsets, n_experts, n_routes,
                                             mean_routes(n_routes, n_experts), d_y, nrows_out, ncols_k, nrows_out,
                                             true, (hipStream_t)stream, d_route_dst)
-                       : launch_gemm_mfma_grouped(d_w_split, d_x_q8_1, d_expert_offsets, n_experts, d_route_dst,
-                                                  d_y, ncols_k, nrows_out, n_routes, (hipStream_t)stream, nullptr,
-                                                  0, true);
+                       : run_grouped(d_w_split, nullptr, 0, d_x_q8_1, d_expert_offsets, n_experts, d_route_dst, d_y,
+                                     ncols_k, nrows_out, n_routes, true, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "grouped gemm (split layout) launch");
     return JJO_OK;
 }
@@ -974,9 +1003,8 @@ int moe_q4_0_gate_up_device(void *stream, const void *w_gate, const void *w_up, 
             ? launch_gemv_routed(w_gate, w_up, x_q8_1_permuted, expert_offsets, num_experts, n_routes,
                                  mean_routes(n_routes, num_experts), gate_up, 2 * intermediate_size, hidden_size,
                                  intermediate_size, false, (hipStream_t)stream)
-            : launch_gemm_mfma_grouped(w_gate, x_q8_1_permuted, expert_offsets, num_experts, nullptr, gate_up,
-                                       hidden_size, 2 * intermediate_size, n_routes, (hipStream_t)stream, w_up,
-                                       intermediate_size);
+            : run_grouped(w_gate, w_up, intermediate_size, x_q8_1_permuted, expert_offsets, num_experts, nullptr,
+                          gate_up, hidden_size, 2 * intermediate_size, n_routes, false, (hipStream_t)stream);
     return e == hipSuccess ? JJO_OK : hip_fail(e, "moe_gate_up launch");
 }
 
@@ -993,9 +1021,8 @@ int moe_q4_0_gate_up_swiglu_q8_1_device(void *stream, const void *w_gate, const 
         return set_error(JJO_ERR_INVALID_ARG, "moe_gate_up_swiglu: intermediate_size must be a multiple of 128");
     if ((rc = check_grouped_grid(n_routes, num_experts)) != JJO_OK) return rc;
     if ((rc = require_gfx950()) != JJO_OK) return rc;
-    hipError_t e = launch_gemm_gate_up_swiglu_q8_1(w_gate, w_up, x_q8_1_permuted, expert_offsets, num_experts,
-                                                   mid_q8_1, hidden_size, intermediate_size, n_routes,
-                                                   (hipStream_t)stream);
+    hipError_t e = run_gate_up_swiglu(w_gate, w_up, x_q8_1_permuted, expert_offsets, num_experts, mid_q8_1,
+                                      hidden_size, intermediate_size, n_routes, false, (hipStream_t)stream);
     return e == hipSuccess ? JJO_OK : hip_fail(e, "moe_gate_up_swiglu launch");
 }
 
@@ -1088,12 +1115,11 @@ int moe_ffn_run(bool split, void *stream, const float *x, const float *logits, c
         return hip_fail(e, "moe_ffn gather");
     // 4) gate|up of every route's expert in one grouped launch whose epilogue applies
     //    SwiGLU and writes the Q8_1 input of the down projection (no fp32 gate|up)
-    if ((e = launch_gemm_gate_up_swiglu_q8_1(w_gate, w_up, ws.xp, ws.offsets, E, ws.midq, H, I, R, s, split)) !=
-        hipSuccess)
+    if ((e = run_gate_up_swiglu(w_gate, w_up, ws.xp, ws.offsets, E, ws.midq, H, I, R, split, s)) != hipSuccess)
         return hip_fail(e, "moe_ffn gate_up_swiglu");
     // 5) down projection, 6) weighted combine back to token order
-    if ((e = launch_gemm_mfma_grouped(w_down, ws.midq, ws.offsets, E, nullptr, ws.eout, I, H, R, s, nullptr, 0,
-                                      split)) != hipSuccess)
+    if ((e = run_grouped(w_down, nullptr, 0, ws.midq, ws.offsets, E, nullptr, ws.eout, I, H, R, split, s)) !=
+        hipSuccess)
         return hip_fail(e, "moe_ffn down");
     if ((e = launch_moe_combine(ws.eout, ws.dst_of_route, ws.route_w, y, T, H, top_k, s)) != hipSuccess)
         return hip_fail(e, "moe_ffn combine");

@@ -39,8 +39,11 @@
 //   * Tile shapes: kslice_pick() below.
 #include <hip/hip_fp16.h>
 
+#include <type_traits>
+
 #include "mfma_q4q8_tile.hpp"
 #include "q4q8_common.hpp"
+#include "q8_1_quant.hpp"
 
 namespace jjo {
 namespace {
@@ -60,57 +63,40 @@ struct KsliceLds {
     static constexpr int kWave = kOffScale + RT * 512;
 };
 
-template <int RT, int CT, int WK, bool SPLIT, int WAVES_PER_SIMD>
-__global__ __launch_bounds__(64 * WK, WAVES_PER_SIMD) void gemm_kslice_kernel(
-    const uint8_t *__restrict__ w, const uint8_t *__restrict__ xq, float *__restrict__ y, int K, int N, int M,
-    int row_tiles, int tok_tiles) {
-    using L = KsliceLds<RT, CT, SPLIT>;
-    extern __shared__ __align__(16) uint8_t smem[];
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int l32 = lane & 31, hh = lane >> 5;
-
-    // Workgroups go round-robin over the 8 XCDs: the token tiles of a row tile follow each
-    // other on one XCD, so its weights come from HBM once.
-    int row_tile = blockIdx.x, tok_tile = 0;
-    if (tok_tiles > 1) {
-        const int slot = blockIdx.x >> 3;
-        row_tile = (slot / tok_tiles) * 8 + (blockIdx.x & 7);
-        tok_tile = slot % tok_tiles;
-        if (row_tile >= row_tiles) return;  // uniform over the workgroup
-    }
-    const int n0 = row_tile * 32 * RT, m0 = tok_tile * 32 * CT;
-    const int nb = K / kQK, nsb = K / kQSuper;
-
-    // ---- staging: rows past N and tokens past M re-read the last valid one ----
-    const uint8_t *wq = w + (size_t)n0 * nb * (SPLIT ? 16 : kQ4BlockBytes);
-    const uint8_t *wd = w + ((size_t)N * 16 + (size_t)n0 * 2) * nb;  // split: the scale plane
-    const uint8_t *xb = xq + (size_t)m0 * kQ8BlockBytes;
-    const size_t x_stride = (size_t)M * kQ8BlockBytes;
-    uint8_t *stage = smem + wave * L::kWave;
-    const uint32_t stage_lds = (uint32_t)(uintptr_t)stage;
-    float *wde = reinterpret_cast<float *>(stage + L::kOffScale);
-    const uint32_t xlim = min(32 * CT, M - m0) * kQ8BlockBytes - 16;
-    uint32_t woff[RT][3];
+// A lane's source offsets of one row tile's weights (first row r0 below the tile's base,
+// `last` the highest valid row there).
+template <bool SPLIT>
+__device__ __forceinline__ void kslice_offsets(uint32_t (&off)[3], int r0, int last, int nb) {
+    const int lane = threadIdx.x & 63;
+    if constexpr (SPLIT) {
+        // lane l: row l/4 of 16, block (l%4) ^ ((row/4)%4): the 16 rows that read one block
+        // then fall in 16 different 16-byte bank groups
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-        const int last = N - 1 - n0;
-        if constexpr (SPLIT) {
-            // lane l: row l/4 of 16, block (l%4) ^ ((row/4)%4): the 16 rows that read one
-            // block then fall in 16 different 16-byte bank groups
+        for (int i = 0; i < 2; ++i)
+            off[i] = (uint32_t)min(r0 + 16 * i + (lane >> 2), last) * nb * 16 + 16 * ((lane & 3) ^ ((lane >> 4) & 3));
+        off[2] = (uint32_t)min(r0 + (lane & 31), last) * nb * 2 + 4 * (lane >> 5);
+    } else {
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
-                woff[rt][i] = (uint32_t)min(32 * rt + 16 * i + (lane >> 2), last) * nb * 16 +
-                              16 * ((lane & 3) ^ ((lane >> 4) & 3));
-            woff[rt][2] = (uint32_t)min(32 * rt + l32, last) * nb * 2 + 4 * hh;
-        } else {
-#pragma unroll
-            for (int i = 0; i < 3; ++i) {
-                const int c = 64 * i + lane;
-                woff[rt][i] = (uint32_t)min(32 * rt + c / 6, last) * nb * kQ4BlockBytes + 12 * (c % 6);
-            }
+        for (int i = 0; i < 3; ++i) {
+            const int c = 64 * i + lane;
+            off[i] = (uint32_t)min(r0 + c / 6, last) * nb * kQ4BlockBytes + 12 * (c % 6);
         }
     }
+}
+
+// One wave's K loop over stages s_beg..s_end-1 of its (32*RT rows) x (32*CT tokens) tile:
+// acc = sum_b d_w/8 * (sumi * d_x) - d_w * s_x (an eighth of the result).  `stage` is the
+// wave's own LDS; rows and tokens past the tile's end re-read the last valid one.
+// wq / wd: per row tile, the weight run (nibble plane when split) and the scale plane at
+// the tile's first row; woff: the lane's byte offsets below them (kslice_offsets).
+template <int RT, int CT, bool SPLIT>
+__device__ __forceinline__ void kslice_loop(f32x16 (&acc)[RT][CT], uint8_t *stage, const uint8_t *const (&wq)[RT],
+                                            const uint8_t *const (&wd)[RT], const uint32_t (&woff)[RT][3],
+                                            const uint8_t *xb, size_t x_stride, uint32_t xlim, int s_beg, int s_end) {
+    using L = KsliceLds<RT, CT, SPLIT>;
+    const int lane = threadIdx.x & 63, l32 = lane & 31, hh = lane >> 5;
+    const uint32_t stage_lds = (uint32_t)(uintptr_t)stage;
+    float *wde = reinterpret_cast<float *>(stage + L::kOffScale);
     // Inline asm: the compiler would order every later LDS access behind these; their
     // completion is waited for at the top of a stage.
     auto dma = [&](int s) {
@@ -133,17 +119,17 @@ __global__ __launch_bounds__(64 * WK, WAVES_PER_SIMD) void gemm_kslice_kernel(
                 if constexpr (!SPLIT)
                     asm volatile("global_load_lds_dwordx3 %0, %1"
                                  :
-                                 : "v"(woff[rt][i]), "s"(wq + (size_t)s * (4 * kQ4BlockBytes)), "{m0}"(m0v)
+                                 : "v"(woff[rt][i]), "s"(wq[rt] + (size_t)s * (4 * kQ4BlockBytes)), "{m0}"(m0v)
                                  : "memory");
                 else if (i < 2)
                     asm volatile("global_load_lds_dwordx4 %0, %1"
                                  :
-                                 : "v"(woff[rt][i]), "s"(wq + (size_t)s * 64), "{m0}"(m0v)
+                                 : "v"(woff[rt][i]), "s"(wq[rt] + (size_t)s * 64), "{m0}"(m0v)
                                  : "memory");
                 else
                     asm volatile("global_load_lds_dword %0, %1"
                                  :
-                                 : "v"(woff[rt][i]), "s"(wd + (size_t)s * 8), "{m0}"(m0v)
+                                 : "v"(woff[rt][i]), "s"(wd[rt] + (size_t)s * 8), "{m0}"(m0v)
                                  : "memory");
             }
         }
@@ -153,7 +139,6 @@ __global__ __launch_bounds__(64 * WK, WAVES_PER_SIMD) void gemm_kslice_kernel(
 #pragma unroll
     for (int v = 0; v < 16; ++v) bias[v] = (int32_t)kBiasBits;
     asm volatile("" : "+v"(bias));
-    f32x16 acc[RT][CT];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
@@ -165,7 +150,6 @@ __global__ __launch_bounds__(64 * WK, WAVES_PER_SIMD) void gemm_kslice_kernel(
     // first half-wave swap completes blocks 0 and 2, the second blocks 1 and 3.
     constexpr int kOrder[4] = {0, 2, 1, 3};
     constexpr int kJobs = 4 * RT * CT;  // 32x32 blocks of a stage
-    const int s_beg = (int)((int64_t)wave * nsb / WK), s_end = (int)((int64_t)(wave + 1) * nsb / WK);
     if (s_beg < s_end) dma(s_beg);
     for (int s = s_beg; s < s_end; ++s) {
         JJO_GEMM_VMCNT(0);  // stage s has landed
@@ -279,6 +263,41 @@ __global__ __launch_bounds__(64 * WK, WAVES_PER_SIMD) void gemm_kslice_kernel(
             }
         }
     }
+}
+
+template <int RT, int CT, int WK, bool SPLIT, int WAVES_PER_SIMD>
+__global__ __launch_bounds__(64 * WK, WAVES_PER_SIMD) void gemm_kslice_kernel(
+    const uint8_t *__restrict__ w, const uint8_t *__restrict__ xq, float *__restrict__ y, int K, int N, int M,
+    int row_tiles, int tok_tiles) {
+    using L = KsliceLds<RT, CT, SPLIT>;
+    extern __shared__ __align__(16) uint8_t smem[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+    // Workgroups go round-robin over the 8 XCDs: the token tiles of a row tile follow each
+    // other on one XCD, so its weights come from HBM once.
+    int row_tile = blockIdx.x, tok_tile = 0;
+    if (tok_tiles > 1) {
+        const int slot = blockIdx.x >> 3;
+        row_tile = (slot / tok_tiles) * 8 + (blockIdx.x & 7);
+        tok_tile = slot % tok_tiles;
+        if (row_tile >= row_tiles) return;  // uniform over the workgroup
+    }
+    const int n0 = row_tile * 32 * RT, m0 = tok_tile * 32 * CT;
+    const int nb = K / kQK, nsb = K / kQSuper;
+
+    f32x16 acc[RT][CT];
+    const uint8_t *wq[RT], *wd[RT];
+    uint32_t woff[RT][3];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        wq[rt] = w + (size_t)n0 * nb * (SPLIT ? 16 : kQ4BlockBytes);
+        wd[rt] = w + ((size_t)N * 16 + (size_t)n0 * 2) * nb;  // split: the scale plane
+        kslice_offsets<SPLIT>(woff[rt], 32 * rt, N - 1 - n0, nb);
+    }
+    kslice_loop<RT, CT, SPLIT>(acc, smem + wave * L::kWave, wq, wd, woff, xq + (size_t)m0 * kQ8BlockBytes,
+                               (size_t)M * kQ8BlockBytes, min(32 * CT, M - m0) * kQ8BlockBytes - 16,
+                               (int)((int64_t)wave * nsb / WK), (int)((int64_t)(wave + 1) * nsb / WK));
 
     // ---- add the K slices in slice order, y[m][n] = 8 * sum ----
     __syncthreads();  // every wave is done with its staging area
@@ -312,6 +331,159 @@ __global__ __launch_bounds__(64 * WK, WAVES_PER_SIMD) void gemm_kslice_kernel(
                 if (n + k < N) yr[k] = v[k];
         }
     }
+}
+
+// ---- grouped (MoE) form: workgroups over (64-row tile, token tile of an expert) ----
+// Token tiles of 32*CT routes, listed expert by expert; a tile with at most 32 routes runs
+// the one-column loop.  kSwiglu: row tile x is gate rows 32x..32x+31 (first row tile) and up
+// rows 32x..32x+31 (second), and instead of storing them the workgroup writes the Q8_1
+// bytes of silu(gate) * up of those 32 intermediate values: one Q8_1 group per route.
+// Every output element is summed in the same order in all of these forms (K slices of the
+// same waves, the same order inside a slice).
+template <int CT, int WK, bool SPLIT, bool kSwiglu>
+__global__ __launch_bounds__(64 * WK, 2) void gemm_kslice_grouped_kernel(
+    const uint8_t *__restrict__ w, const uint8_t *__restrict__ w2, const uint8_t *__restrict__ xq,
+    float *__restrict__ y, uint8_t *__restrict__ midq, int K, int N, int M, int n_split,
+    const int32_t *__restrict__ expert_offsets, int n_experts, const int32_t *__restrict__ route_dst) {
+    constexpr int RT = 2;
+    extern __shared__ __align__(16) uint8_t smem[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nb = K / kQK, nsb = K / kQSuper;
+
+    // Tile blockIdx.y of the concatenated per-expert tile lists, 64 experts per step.
+    // Ranges are clamped to [0, M]: a malformed table drops routes, it reads nothing outside.
+    int t = blockIdx.y, m0 = -1, m_end = 0, expert = 0;
+    for (int e0 = 0; e0 < n_experts && m0 < 0; e0 += 64) {
+        const int ei = e0 + lane;
+        int beg = 0, end = 0;
+        if (ei < n_experts) {
+            beg = min(max(expert_offsets[ei], 0), M);
+            end = min(max(expert_offsets[ei + 1], beg), M);
+        }
+        const int tiles = (end - beg + 32 * CT - 1) / (32 * CT);
+        int incl = tiles;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int o = __shfl_up(incl, d);
+            if (lane >= d) incl += o;
+        }
+        const int total = __shfl(incl, 63);
+        if (t < total) {
+            const int f = __builtin_ctzll(__ballot(incl > t));  // the expert holding tile t
+            m0 = __shfl(beg, f) + (t - (__shfl(incl, f) - __shfl(tiles, f))) * (32 * CT);
+            m_end = __shfl(end, f);
+            expert = e0 + f;
+        } else {
+            t -= total;
+        }
+    }
+    if (m0 < 0) return;  // uniform over the workgroup
+    m0 = __builtin_amdgcn_readfirstlane(m0);
+    m_end = __builtin_amdgcn_readfirstlane(m_end);
+    expert = __builtin_amdgcn_readfirstlane(expert);
+
+    // Row tile rt: rows r0.. of one matrix with `rows_e` rows per expert (n_split % 64 == 0,
+    // so a 64-row tile of two stacked matrices lies in one of them).
+    const uint8_t *wq[RT], *wd[RT];
+    uint32_t woff[RT][3];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        const uint8_t *mat = w;
+        int rows_e = N, r0 = blockIdx.x * 64 + 32 * rt;
+        if constexpr (kSwiglu) {
+            mat = rt == 0 ? w : w2;
+            rows_e = n_split;
+            r0 = blockIdx.x * 32;
+        } else if (w2 != nullptr) {
+            const bool second = r0 >= n_split;
+            mat = second ? w2 : w;
+            rows_e = second ? N - n_split : n_split;
+            r0 -= second ? n_split : 0;
+        }
+        const size_t row = (size_t)expert * rows_e + min(r0, rows_e - 1);
+        wq[rt] = mat + row * nb * (SPLIT ? 16 : kQ4BlockBytes);
+        wd[rt] = mat + ((size_t)n_experts * rows_e * 16 + row * 2) * nb;  // split: the scale plane
+        kslice_offsets<SPLIT>(woff[rt], 0, max(rows_e - 1 - r0, 0), nb);
+    }
+    const uint8_t *xb = xq + (size_t)m0 * kQ8BlockBytes;
+    const size_t x_stride = (size_t)M * kQ8BlockBytes;
+    const int s_beg = (int)((int64_t)wave * nsb / WK), s_end = (int)((int64_t)(wave + 1) * nsb / WK);
+    f32x4 *red = reinterpret_cast<f32x4 *>(smem);
+
+    auto run = [&](auto ct_tag) {
+        constexpr int C = decltype(ct_tag)::value;
+        const int valid = min(32 * C, m_end - m0);
+        f32x16 acc[RT][C];
+        kslice_loop<RT, C, SPLIT>(acc, smem + wave * KsliceLds<RT, C, SPLIT>::kWave, wq, wd, woff, xb, x_stride,
+                                  valid * kQ8BlockBytes - 16, s_beg, s_end);
+        __syncthreads();  // every wave is done with its staging area
+        constexpr int kTile = C * 256, kItems = RT * kTile;
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+            for (int ct = 0; ct < C; ++ct)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    red[wave * kItems + (rt * C + ct) * 256 + q * 64 + lane] = f32x4{
+                        acc[rt][ct][4 * q], acc[rt][ct][4 * q + 1], acc[rt][ct][4 * q + 2], acc[rt][ct][4 * q + 3]};
+        __syncthreads();
+        auto sum = [&](int src) {
+            f32x4 v = red[src];
+#pragma unroll
+            for (int i = 1; i < WK; ++i) v += red[i * kItems + src];
+            return v * 8.0f;
+        };
+        // Eight consecutive threads take the 32 rows of one token.
+        for (int it = tid; it < (kSwiglu ? kTile : kItems); it += 64 * WK) {
+            const int qh = it & 7, tok = (it >> 3) & 31, tile = it >> 8;
+            const int src = tile * 256 + (qh >> 1) * 64 + tok + 32 * (qh & 1);
+            const int m = m0 + 32 * (tile % C) + tok;
+            if constexpr (kSwiglu) {
+                const f32x4 g = sum(src), u = sum(kTile + src);
+                uint32_t ds;  // every lane of the wave is active here (the group butterfly)
+                const uint32_t qv = quantize_group8(swiglu(g.x, u.x), swiglu(g.y, u.y), swiglu(g.z, u.z),
+                                                    swiglu(g.w, u.w), &ds);
+                if (m < m_end) {
+                    const int grp = blockIdx.x & 3;  // 32-group of the superblock
+                    uint8_t *blk = midq + ((size_t)(blockIdx.x >> 2) * M + m) * kQ8BlockBytes;
+                    *reinterpret_cast<uint32_t *>(blk + 16 + 32 * grp + 4 * qh) = qv;
+                    if (qh == 0) *reinterpret_cast<uint32_t *>(blk + 4 * grp) = ds;
+                }
+            } else if (m < m_end) {
+                const f32x4 v = sum(src);
+                const int n = blockIdx.x * 64 + 32 * (tile / C) + 4 * qh;
+                float *yr = y + (size_t)(route_dst != nullptr ? route_dst[m] : m) * N + n;
+                if (n + 3 < N && (N & 3) == 0) {
+                    *reinterpret_cast<f32x4 *>(yr) = v;
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        if (n + k < N) yr[k] = v[k];
+                }
+            }
+        }
+    };
+    if (CT == 1 || m_end - m0 <= 32)
+        run(std::integral_constant<int, 1>{});
+    else
+        run(std::integral_constant<int, CT>{});
+}
+
+template <int CT, int WK, bool SPLIT, bool kSwiglu>
+hipError_t launch_grouped(const void *w, const void *w2, const void *xq, float *y, void *midq, int K, int N, int M,
+                          int n_split, const int32_t *offsets, int n_experts, const int32_t *route_dst,
+                          hipStream_t stream) {
+    auto kern = gemm_kslice_grouped_kernel<CT, WK, SPLIT, kSwiglu>;
+    const size_t stage = WK * (size_t)KsliceLds<2, CT, SPLIT>::kWave, red = (size_t)WK * 2 * CT * 4096;
+    const size_t lds = stage > red ? stage : red;
+    hipError_t e = ensure_dynamic_lds((const void *)kern, lds);
+    if (e != hipSuccess) return e;
+    // Upper bound on the token tiles over all experts.
+    const dim3 grid(kSwiglu ? n_split / 32 : (N + 63) / 64, (M + 32 * CT - 1) / (32 * CT) + n_experts);
+    hipLaunchKernelGGL(kern, grid, dim3(64 * WK), lds, stream, (const uint8_t *)w, (const uint8_t *)w2,
+                       (const uint8_t *)xq, y, (uint8_t *)midq, K, N, M, n_split, offsets, n_experts, route_dst);
+    return hipGetLastError();
 }
 
 template <int RT, int CT, int WK, int WAVES_PER_SIMD>
@@ -369,6 +541,26 @@ hipError_t launch_gemm_kslice(const void *w, const void *xq, float *y, int K, in
         case 2: return launch<2, 2, 8, 2>(w, xq, y, K, N, M, split, stream);
         default: return launch<2, 2, 4, 2>(w, xq, y, K, N, M, split, stream);
     }
+}
+
+hipError_t launch_gemm_kslice_grouped(const void *w, const void *w2, const void *xq, float *y, void *midq, int K,
+                                      int N, int M, int n_split, const int32_t *offsets, int n_experts,
+                                      const int32_t *route_dst, bool split, int cols, hipStream_t stream) {
+    // Four waves: two (64 routes) or three (32 routes) workgroups share a CU, and an
+    // expert's ragged last tile ends sooner than with eight (E=64 top-8, 100 tokens, FFN:
+    // 137 us against 195).
+    auto go = [&](auto ct, auto sp, auto sw) {
+        return launch_grouped<decltype(ct)::value, 4, decltype(sp)::value, decltype(sw)::value>(
+            w, w2, xq, y, midq, K, N, M, n_split, offsets, n_experts, route_dst, stream);
+    };
+    auto with_layout = [&](auto ct, auto sw) {
+        return split ? go(ct, std::true_type{}, sw) : go(ct, std::false_type{}, sw);
+    };
+    auto with_cols = [&](auto sw) {
+        return cols == 1 ? with_layout(std::integral_constant<int, 1>{}, sw)
+                         : with_layout(std::integral_constant<int, 2>{}, sw);
+    };
+    return midq != nullptr ? with_cols(std::true_type{}) : with_cols(std::false_type{});
 }
 
 }  // namespace jjo

@@ -95,6 +95,12 @@ hipError_t launch_gemm_mfma64(const void *w, const void *xq, float *y, int K, in
 int kslice_pick(int K, int N, int M, double *us);
 hipError_t launch_gemm_kslice(const void *w, const void *xq, float *y, int K, int N, int M, bool split, int shape,
                               hipStream_t stream);
+// Its grouped form (experts' row tiles x tiles of 32 * cols routes, cols 1 or 2).  midq == nullptr: the
+// products (w2: a second stacked matrix, columns n_split.. of y; n_split % 64 == 0);
+// midq: the Q8_1 bytes of silu(gate) * up, w = gate, w2 = up, n_split = their rows.
+hipError_t launch_gemm_kslice_grouped(const void *w, const void *w2, const void *xq, float *y, void *midq, int K,
+                                      int N, int M, int n_split, const int32_t *offsets, int n_experts,
+                                      const int32_t *route_dst, bool split, int cols, hipStream_t stream);
 hipError_t launch_gemm_mfma(const void *w, const void *xq, float *y, int K, int N, int M,
                             hipStream_t stream);
 hipError_t launch_gemm_mfma_grouped(const void *w, const void *xq, const int32_t *expert_offsets,

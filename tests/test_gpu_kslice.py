@@ -72,3 +72,41 @@ def test_kslice_special_scales(dev):
     assert np.isnan(got[7]).all() and np.isnan(exp[7]).all()
     rest = [m for m in range(M) if m != 7]
     np.testing.assert_allclose(got[rest], exp[rest], rtol=RTOL, atol=ATOL)
+
+
+@pytest.mark.parametrize("counts,N,K", [
+    # one column tile (mean of at most 24 routes per expert): full, tail, empty and single-route experts
+    ([32, 0, 1, 33, 31, 5, 64], 96, 384), ([20] * 3, 65, 128), ([2] * 30 + [70], 257, 1152),
+    # two column tiles, tails that run the one-column loop
+    ([64, 65, 1, 0, 96, 97, 32, 33], 130, 640), ([128, 31], 64, 256),
+])
+def test_kslice_grouped(counts, N, K, dev):
+    """The grouped form at its tile edges, scattered outputs, both layouts (equal bits)."""
+    import torch
+    E, R = len(counts), sum(counts)
+    assert R > 48  # below, the grouped entry is a GEMV
+    print(f"[case] kslice grouped E={E} R={R} N={N} K={K}", flush=True)
+    rng = np.random.default_rng(R + N)
+    ws = [c_oracle.quantize_q4_0((rng.standard_normal((N, K)) * 0.02).astype(np.float32)) for _ in counts]
+    xq = c_oracle.quantize_q8_1(rng.standard_normal((R, K)).astype(np.float32), [K, R])
+    off = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    dst = rng.permutation(R).astype(np.int32)
+    exp = np.empty((R, N), np.float32)
+    blocks = xq.reshape(K // 128, R, 144)
+    for e, n in enumerate(counts):
+        if n:
+            rows = np.ascontiguousarray(blocks[:, off[e]:off[e + 1]]).reshape(-1)
+            exp[dst[off[e]:off[e + 1]]] = c_oracle.matmul(ws[e], rows, K, N, n)
+    w = torch.from_numpy(np.concatenate(ws)).to(dev)
+    w_split = torch.empty_like(w)
+    capi.q4_0_to_split(w, w_split, E * N, K)
+    got = []
+    for split in (False, True):
+        y = torch.full((R * N + 64,), float("nan"), dtype=torch.float32, device=dev)
+        capi.grouped_mat_mul(w_split if split else w, torch.from_numpy(xq).to(dev), torch.from_numpy(off).to(dev), y, K,
+                             N, R, route_dst=torch.from_numpy(dst).to(dev), split=split)
+        torch.cuda.synchronize()
+        assert torch.isnan(y[R * N:]).all()
+        got.append(y[:R * N].cpu().numpy().reshape(R, N))
+        np.testing.assert_allclose(got[-1], exp, rtol=RTOL, atol=ATOL)
+    assert np.array_equal(got[0], got[1])
