@@ -3,6 +3,7 @@
 Outputs (next to this file):
   libjjjetson_ops_amd.so             HIP kernels + C ABI (hipcc, gfx950 only)
   q8_1_me<ext>.so, mm_q4_0_q8_1_me<ext>.so   pybind11 modules linked to it
+  _linear<ext>.so                    CPython binding of the linear-layer entries
 
 Run:  python -m jjjetson_ops_amd.build      (or call build_all()).
 """
@@ -39,7 +40,8 @@ HIP_FLAGS = [
     f"-I{INCLUDE}",
     f"-I{CSRC}",
 ]
-PYBIND_MODULES = {"q8_1_me": "bind_q8_1.cpp", "mm_q4_0_q8_1_me": "bind_mm_q4_0_q8_1.cpp"}
+PYBIND_MODULES = {"q8_1_me": "bind_q8_1.cpp", "mm_q4_0_q8_1_me": "bind_mm_q4_0_q8_1.cpp",
+                  "_linear": "bind_linear.cpp"}
 
 
 def _run(cmd: list[str]) -> None:

@@ -226,21 +226,45 @@ def q8_1_output_bytes(dims) -> int:
     return int(lib().q8_1_output_bytes(d, n))
 
 
-def _stream(stream):
-    if stream is None:
+_torch = None
+
+
+def _current_stream() -> int:
+    """The current torch stream of the current device, as an address."""
+    global _torch
+    if _torch is None:
         import torch
-        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        _torch = torch
+    return _torch._C._cuda_getCurrentRawStream(_torch.cuda.current_device())
+
+
+def _stream(stream) -> int:
+    if stream is None:
+        return _current_stream()
     if isinstance(stream, int):
-        return ctypes.c_void_p(stream)
-    return ctypes.c_void_p(stream.cuda_stream)
+        return stream
+    return stream.cuda_stream
 
 
-def _dev(t, name: str):
+def _dev(t, name: str) -> int:
     if not t.is_cuda:
         raise ValueError(f"{name} must be a device tensor")
     if not t.is_contiguous():
         raise ValueError(f"{name} must be contiguous")
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()
+
+
+_linear_native = None
+
+
+def _linear(split: bool, x, w, y, in_features, out_features, num_tokens, ws, stream) -> int:
+    """The two linear entries through the native binding (csrc/bind_linear.cpp)."""
+    global _linear_native
+    if _linear_native is None:
+        lib()  # the same loud failure where nothing is built
+        from ._linear import linear
+        _linear_native = linear
+    return _linear_native(split, _current_stream, x, w, y, in_features, out_features, num_tokens, ws, stream)
 
 
 def quantize_q8_1(x, out, dims=None, stream=None) -> None:
@@ -399,18 +423,17 @@ def parse_q8_1(raw, n_blocks: int):
 # ---------------------------------------------------------------- engine linear
 def linear_q4_0(x, w, y, in_features: int, out_features: int, num_tokens: int, ws=None, stream=None) -> None:
     """linear_q4_0_forward_device: y [T, out] = x [T, in] . dequant(w [out, in/32 blocks]).T"""
-    _check(lib().linear_q4_0_forward_device(_stream(stream), None if ws is None else _dev(ws, "ws"), _dev(x, "x"),
-                                            _dev(w, "w"), _dev(y, "y"), in_features, out_features, num_tokens),
-           "linear_q4_0_forward_device")
+    rc = _linear(False, x, w, y, in_features, out_features, num_tokens, ws, stream)
+    if rc != JJO_OK:
+        _check(rc, "linear_q4_0_forward_device")
 
 
 def linear_q4_0_split(x, ws_split, y, in_features: int, out_features: int, num_tokens: int, ws=None,
                       stream=None) -> None:
     """linear_q4_0s_forward_device: linear_q4_0 on weights repacked into the split layout."""
-    _check(lib().linear_q4_0s_forward_device(_stream(stream), None if ws is None else _dev(ws, "ws"), _dev(x, "x"),
-                                             _dev(ws_split, "w"), _dev(y, "y"), in_features, out_features,
-                                             num_tokens),
-           "linear_q4_0s_forward_device")
+    rc = _linear(True, x, ws_split, y, in_features, out_features, num_tokens, ws, stream)
+    if rc != JJO_OK:
+        _check(rc, "linear_q4_0s_forward_device")
 
 
 def linear_q4_0_noalloc(x, w, y, in_features: int, out_features: int, num_tokens: int, stream=None) -> None:
