@@ -274,15 +274,13 @@ __global__ __launch_bounds__(64 * WK, WAVES_PER_SIMD) void gemm_kslice_kernel(
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
-    // Workgroups go round-robin over the 8 XCDs: the token tiles of a row tile follow each
-    // other on one XCD, so its weights come from HBM once.
-    int row_tile = blockIdx.x, tok_tile = 0;
-    if (tok_tiles > 1) {
-        const int slot = blockIdx.x >> 3;
-        row_tile = (slot / tok_tiles) * 8 + (blockIdx.x & 7);
-        tok_tile = slot % tok_tiles;
-        if (row_tile >= row_tiles) return;  // uniform over the workgroup
-    }
+    // Workgroups go round-robin over the 8 XCDs: each XCD takes one contiguous eighth of the
+    // tiles, the token tiles of a row tile following each other, so its weights come from
+    // HBM (nearly) once and no XCD gets more than one tile above the mean.
+    const int tiles = row_tiles * tok_tiles, per_xcd = (tiles + 7) >> 3;
+    const int tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (tile >= tiles) return;  // uniform over the workgroup
+    const int row_tile = tile / tok_tiles, tok_tile = tile % tok_tiles;
     const int n0 = row_tile * 32 * RT, m0 = tok_tile * 32 * CT;
     const int nb = K / kQK, nsb = K / kQSuper;
 
@@ -495,25 +493,26 @@ hipError_t launch(const void *w, const void *xq, float *y, int K, int N, int M, 
     hipError_t e = ensure_dynamic_lds((const void *)kern, lds);
     if (e != hipSuccess) return e;
     const int64_t rows = ((int64_t)N + 32 * RT - 1) / (32 * RT), toks = ((int64_t)M + 32 * CT - 1) / (32 * CT);
-    const int64_t grid = toks == 1 ? rows : (rows + 7) / 8 * 8 * toks;
+    const int64_t grid = (rows * toks + 7) / 8 * 8;
     if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * WK), lds, stream, (const uint8_t *)w,
                        (const uint8_t *)xq, y, K, N, M, (int)rows, (int)toks);
     return hipGetLastError();
 }
 
-// The tile shapes, with the time one CU takes for a 128-value stage of one workgroup's
-// tile (us, measured at K=4096, 11008 and 14336 with N=2048..14336 and 24..1024 tokens),
-// with its slots full and with a single workgroup on the CU.
+// The tile shapes with their estimated time: a launch runs in rounds of `resident`
+// workgroups per CU; a round costs round_us + stage_us per 128-value stage, a (last) round
+// of at most one workgroup per CU alone_us per stage.  Fitted to K=1024..14336, N=1024..14336,
+// 17..1024 tokens, both layouts; within about 10% of the measurements.
 struct Shape {
-    int rt, ct;
-    double us, us_alone;
+    int rt, ct, resident;
+    double fixed_us, round_us, stage_us, alone_us;
 };
 constexpr Shape kShapes[] = {
-    {1, 1, 0.14, 0.14},  // 8 waves, two workgroups per CU
-    {1, 2, 0.25, 0.25},  // 8 waves, one workgroup per CU
-    {2, 2, 0.46, 0.46},  // 8 waves, one workgroup per CU
-    {2, 2, 0.42, 0.51},  // 4 waves, two workgroups per CU
+    {1, 1, 2, 3.5, 0.5, 0.300, 0.185},  // 8 waves (N=4096, K=4096, 64 tokens: 8.4 us)
+    {1, 2, 1, 2.0, 3.2, 0.210, 0.210},  // 8 waves (100 tokens: 11.9)
+    {2, 2, 1, 2.0, 3.0, 0.420, 0.420},  // 8 waves (256 tokens: 18.5)
+    {2, 2, 2, 3.0, 3.2, 0.775, 0.530},  // 4 waves (512 tokens: 30.7)
 };
 
 }  // namespace
@@ -524,7 +523,10 @@ int kslice_pick(int K, int N, int M, double *us) {
     for (int i = 0; i < (int)(sizeof(kShapes) / sizeof(kShapes[0])); ++i) {
         const Shape &s = kShapes[i];
         const int64_t g = (((int64_t)N + 32 * s.rt - 1) / (32 * s.rt)) * (((int64_t)M + 32 * s.ct - 1) / (32 * s.ct));
-        const double t = 3.5 + (K / kQSuper) * (double)((g + cus - 1) / cus) * (g > cus ? s.us : s.us_alone);
+        const int64_t slots = s.resident * cus, rem = g % slots;
+        const double stages = K / kQSuper, round = s.round_us + s.stage_us * stages;
+        const double t = s.fixed_us + (double)(g / slots) * round +
+                         (rem == 0 ? 0.0 : rem > cus ? round : s.round_us + s.alone_us * stages);
         if (i == 0 || t < *us) {
             best = i;
             *us = t;
