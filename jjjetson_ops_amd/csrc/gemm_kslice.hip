@@ -321,8 +321,8 @@ __global__ __launch_bounds__(64 * WK, WAVES_PER_SIMD) void gemm_kslice_kernel(
         const int m = m0 + 32 * (tile % CT) + tok, n = n0 + 32 * (tile / CT) + 4 * qh;
         if (m >= M) continue;
         float *yr = y + (size_t)m * N + n;
-        if (n + 3 < N && (N & 3) == 0) {
-            *reinterpret_cast<f32x4 *>(yr) = v;
+        if (n + 3 < N) {
+            *reinterpret_cast<f32x4a4 *>(yr) = v;
         } else {
 #pragma unroll
             for (int k = 0; k < 4; ++k)
@@ -452,8 +452,8 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_kslice_grouped_kernel(
                 const f32x4 v = sum(src);
                 const int n = blockIdx.x * 64 + 32 * (tile / C) + 4 * qh;
                 float *yr = y + (size_t)(route_dst != nullptr ? route_dst[m] : m) * N + n;
-                if (n + 3 < N && (N & 3) == 0) {
-                    *reinterpret_cast<f32x4 *>(yr) = v;
+                if (n + 3 < N) {
+                    *reinterpret_cast<f32x4a4 *>(yr) = v;
                 } else {
 #pragma unroll
                     for (int k = 0; k < 4; ++k)

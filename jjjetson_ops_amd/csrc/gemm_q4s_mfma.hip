@@ -299,8 +299,8 @@ __global__ __launch_bounds__(g2::kThreads, 2) void gemm_q4s_mfma_kernel(const ui
                 const float v1 = 8.0f * acc[ct][4 * q + 1];
                 const float v2 = 8.0f * acc[ct][4 * q + 2];
                 const float v3 = 8.0f * acc[ct][4 * q + 3];
-                if (n + 3 < N && (N & 3) == 0) {
-                    *reinterpret_cast<float4 *>(yrow + n) = make_float4(v0, v1, v2, v3);
+                if (n + 3 < N) {
+                    *reinterpret_cast<f32x4a4 *>(yrow + n) = f32x4a4{v0, v1, v2, v3};
                 } else {
                     if (n + 0 < N) yrow[n + 0] = v0;
                     if (n + 1 < N) yrow[n + 1] = v1;

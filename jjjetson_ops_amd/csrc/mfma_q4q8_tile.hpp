@@ -22,6 +22,10 @@ typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
 typedef int32_t i32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+// Four consecutive outputs of a row of y: rows are only 4-byte aligned when N % 4 != 0, and
+// a 4-byte-aligned 16-byte store costs what an aligned one does (four single stores:
+// N=2151, K=3072, 1894 tokens 57.9 us against 49.6 at N=2152).
+typedef float f32x4a4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));           // 16-B aligned
