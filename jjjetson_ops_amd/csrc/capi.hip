@@ -186,7 +186,7 @@ int small_tile_rows(int N, int M) {
 // 11.8, 512: 37.4 / 31.1, 2048: 105-110 / 112 (stays tiled); K=11008: 48: 52 / 18, 1024:
 // 157-167 / 140; N=14336, K=4096: 100: 37.6 / 31, 512: 105-117 / 98, 1024: 197 / 197.
 int kslice_shape(int K, int N, int M) {
-    if (M > 65535) return -1;
+    if (M > 65535 || K >= kMaxTileK) return -1;
     const double stages = K / kQSuper, cus = device_cus();
     double tiled;
     if (const int tr = small_tile_rows(N, M); tr != 0) {
@@ -579,7 +579,8 @@ int mean_routes(int n_routes, int n_experts) {
 // / 243, 25: 323 -> 248 / 262, 32: 475 -> 375 / 313, 64: 554 -> 542 / 488, 128: 798 -> 928 /
 // 804.  The mean hides the skew of a random router: from about 24 on, most launches hold
 // an expert above 32 routes, whose weights one column tile reads twice.
-int grouped_kslice_cols(int n_routes, int n_experts) {
+int grouped_kslice_cols(int n_routes, int n_experts, int K) {
+    if (K >= kMaxTileK) return 0;
     const int mean = mean_routes(n_routes, n_experts);
     return mean <= 24 ? 1 : mean <= 80 ? 2 : 0;
 }
@@ -587,7 +588,7 @@ int grouped_kslice_cols(int n_routes, int n_experts) {
 hipError_t run_grouped(const void *w, const void *w2, int n_split, const void *xq, const int32_t *offsets,
                        int n_experts, const int32_t *route_dst, float *y, int K, int N, int n_routes, bool split,
                        hipStream_t s) {
-    if (const int cols = grouped_kslice_cols(n_routes, n_experts); cols > 0)
+    if (const int cols = grouped_kslice_cols(n_routes, n_experts, K); cols > 0)
         return launch_gemm_kslice_grouped(w, w2, xq, y, nullptr, K, N, n_routes, n_split, offsets, n_experts,
                                           route_dst, split, cols, s);
     return launch_gemm_mfma_grouped(w, xq, offsets, n_experts, route_dst, y, K, N, n_routes, s, w2, n_split, split);
@@ -595,7 +596,7 @@ hipError_t run_grouped(const void *w, const void *w2, int n_split, const void *x
 
 hipError_t run_gate_up_swiglu(const void *w_gate, const void *w_up, const void *xq, const int32_t *offsets,
                               int n_experts, void *mid_q8_1, int K, int I, int n_routes, bool split, hipStream_t s) {
-    if (const int cols = grouped_kslice_cols(n_routes, n_experts); cols > 0)
+    if (const int cols = grouped_kslice_cols(n_routes, n_experts, K); cols > 0)
         return launch_gemm_kslice_grouped(w_gate, w_up, xq, nullptr, mid_q8_1, K, 2 * I, n_routes, I, offsets,
                                           n_experts, nullptr, split, cols, s);
     return launch_gemm_gate_up_swiglu_q8_1(w_gate, w_up, xq, offsets, n_experts, mid_q8_1, K, I, n_routes, s, split);

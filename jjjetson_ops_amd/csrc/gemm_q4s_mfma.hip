@@ -30,7 +30,10 @@
 //     superblock are one contiguous 18 KB run, copied to LDS by LDS DMA.
 //   * Double-buffered LDS (29 KB per stage), one barrier per stage, two
 //     workgroups per CU: the two waves of a SIMD belong to different workgroups,
-//     so one's barrier wait does not stall the other.
+//     so one's barrier wait does not stall the other.  The next stage's loads are
+//     spread over the blocks of this one (M=2048, K=4096, split: N=14336 363 -> 349 us,
+//     N=4096 109 -> 99).  At N=14336 the chip runs this kernel at about 1.7 GHz (power),
+//     so what is left is instructions and LDS bytes, not waits.
 #include <hip/hip_fp16.h>
 
 #include <type_traits>
@@ -85,6 +88,7 @@ __global__ __launch_bounds__(g2::kThreads, 2) void gemm_q4s_mfma_kernel(const ui
     }
     const int n0 = (tile % n_tiles_n) * BN;
     const int m0 = (tile / n_tiles_n) * BM + (half > 0 ? BM / 2 : 0);
+    if (m0 >= M) return;  // the second half of a tail tile without tokens (uniform)
     const int tile_tokens = half < 0 ? BM : BM / 2;
     const int nb = K / kQK;
     const int n_stages = nb / KB;
@@ -100,15 +104,15 @@ __global__ __launch_bounds__(g2::kThreads, 2) void gemm_q4s_mfma_kernel(const ui
         const int unit = min(wave + 4 * i, kXRuns - 1) * 64 + lane;
         x_off[i] = unit < x_valid_units ? unit * 16 : 0;
     }
-    auto dma_x = [&](int c, int buf) {
+    auto dma_x = [&](int c, int buf, int i0, int i1) {  // 1 KB runs wave + 4i, i0 <= i < i1
         const uint32_t xs = (uint32_t)(uintptr_t)(smem + buf * kBufBytes);
         const uint8_t *src = x_base + (size_t)c * x_stride;
 #pragma unroll
         for (int i = 0; i < 5; ++i) {
+            if (i < i0 || i >= i1) continue;
             const int run = min(wave + 4 * i, kXRuns - 1);
-            if (run * 64 >= x_valid_units) continue;  // wave-uniform
             const uint32_t m0v = __builtin_amdgcn_readfirstlane(xs + run * 1024);
-            asm volatile("global_load_lds_dwordx4 %0, off" : : "v"(src + x_off[i]), "{m0}"(m0v) : "memory");
+            asm volatile("global_load_lds_dwordx4 %0, %1" : : "v"(x_off[i]), "s"(src), "{m0}"(m0v) : "memory");
         }
     };
 
@@ -118,12 +122,14 @@ __global__ __launch_bounds__(g2::kThreads, 2) void gemm_q4s_mfma_kernel(const ui
     // runs of 64 rows x 16 bytes); thread t loads the two fp16 scales of row t/2,
     // blocks 2(t&1), 2(t&1)+1.
     const int st_row = tid >> 1, st_pair = tid & 1;
-    const uint8_t *wq_src0 = w + ((size_t)min(n0 + lane, N - 1) * nb + wave) * 16;
-    const uint8_t *wq_src1 = w + ((size_t)min(n0 + 64 + lane, N - 1) * nb + wave) * 16;
-    const uint32_t *wd_src =
-        reinterpret_cast<const uint32_t *>(w + qs_plane + ((size_t)min(n0 + st_row, N - 1) * nb + 2 * st_pair) * 2);
+    const uint8_t *wq_base = w + ((size_t)n0 * nb + wave) * 16;
+    const uint32_t wq_off0 = (uint32_t)min(lane, N - 1 - n0) * nb * 16;
+    const uint32_t wq_off1 = (uint32_t)min(64 + lane, N - 1 - n0) * nb * 16;
+    const uint8_t *wd_base = w + qs_plane + (size_t)n0 * nb * 2;
+    const uint32_t wd_off = ((uint32_t)min(st_row, N - 1 - n0) * nb + 2 * st_pair) * 2;
     // block_q4_0: thread t holds the 36 bytes of row t/2, blocks 2(t&1), 2(t&1)+1.
-    const uint8_t *wr_src = w + (size_t)min(n0 + st_row, N - 1) * nb * kQ4BlockBytes + st_pair * 36;
+    const uint8_t *wr_base = w + (size_t)n0 * nb * kQ4BlockBytes;
+    const uint32_t wr_off = (uint32_t)min(st_row, N - 1 - n0) * nb * kQ4BlockBytes + st_pair * 36;
     uint32_t wst[SPLIT ? 1 : 9];
 
     auto load_w = [&](int c, int buf) {
@@ -131,13 +137,12 @@ __global__ __launch_bounds__(g2::kThreads, 2) void gemm_q4s_mfma_kernel(const ui
             const uint32_t wqs = (uint32_t)(uintptr_t)(smem + buf * kBufBytes + kOffWq) + wave * (BN * 16);
             const uint32_t m0a = __builtin_amdgcn_readfirstlane(wqs);
             const uint32_t m0b = __builtin_amdgcn_readfirstlane(wqs + 64 * 16);
-            asm volatile("global_load_lds_dwordx4 %0, off" : : "v"(wq_src0 + (size_t)c * (KB * 16)), "{m0}"(m0a)
-                         : "memory");
-            asm volatile("global_load_lds_dwordx4 %0, off" : : "v"(wq_src1 + (size_t)c * (KB * 16)), "{m0}"(m0b)
-                         : "memory");
-            wst[0] = wd_src[c * 2];  // 4 blocks per stage = 8 bytes = 2 dwords per row
+            const uint8_t *src = wq_base + (size_t)c * (KB * 16);
+            asm volatile("global_load_lds_dwordx4 %0, %1" : : "v"(wq_off0), "s"(src), "{m0}"(m0a) : "memory");
+            asm volatile("global_load_lds_dwordx4 %0, %1" : : "v"(wq_off1), "s"(src), "{m0}"(m0b) : "memory");
+            wst[0] = *reinterpret_cast<const uint32_t *>(wd_base + (size_t)c * (KB * 2) + wd_off);
         } else {
-            const uint8_t *p = wr_src + (size_t)c * (KB * kQ4BlockBytes);
+            const uint8_t *p = wr_base + (size_t)c * (KB * kQ4BlockBytes) + wr_off;
             const u32x4a4 a = *reinterpret_cast<const u32x4a4 *>(p);
             const u32x4a4 b = *reinterpret_cast<const u32x4a4 *>(p + 16);
             wst[0] = a.x; wst[1] = a.y; wst[2] = a.z; wst[3] = a.w;
@@ -192,17 +197,13 @@ __global__ __launch_bounds__(g2::kThreads, 2) void gemm_q4s_mfma_kernel(const ui
     for (int v = 0; v < 16; ++v) bias[v] = (int32_t)kBiasBits;
     asm volatile("" : "+v"(bias));
 
-    // ---- prologue: stage 0 into buffer 0, stage 1 in flight into buffer 1 ----
-    dma_x(0, 0);
+    // ---- prologue: stage 0 into buffer 0 ----
     load_w(0, 0);
+    dma_x(0, 0, 0, 5);
     JJO_GEMM_VMCNT(0);
     store_w(0);
     __syncthreads();
     zero_tail_headers(0);
-    if (n_stages > 1) {
-        dma_x(1, 1);
-        load_w(1, 1);
-    }
 
     auto run = [&](auto ct_tag) {
         constexpr int CT = decltype(ct_tag)::value;  // 32-token column tiles of this tile
@@ -213,7 +214,9 @@ __global__ __launch_bounds__(g2::kThreads, 2) void gemm_q4s_mfma_kernel(const ui
             for (int v = 0; v < 16; ++v) acc[ct][v] = 0.0f;
         const int shift = 4 * hh;
         for (int c = 0; c < n_stages; ++c) {
-            const int buf = c & 1;
+            // The last stage loads itself again (into a buffer nobody reads): a branch around
+            // the loads would split the unrolled blocks (it spilled 420 bytes per lane).
+            const int buf = c & 1, c1 = min(c + 1, n_stages - 1);
             const uint8_t *xs = smem + buf * kBufBytes;
             const uint8_t *wqs = xs + kOffWq;
             const float *wde = reinterpret_cast<const float *>(xs + kOffWde);
@@ -227,6 +230,12 @@ __global__ __launch_bounds__(g2::kThreads, 2) void gemm_q4s_mfma_kernel(const ui
             }
 #pragma unroll
             for (int b = 0; b < KB; ++b) {
+                // Stage c+1 goes into the other buffer (which no wave reads until the barrier
+                // below) a few instructions per block: issued in one burst after the barrier
+                // by all four waves they queued for 620 of a stage's 5390 clocks.
+                if (b == 0) load_w(c1, buf ^ 1);
+                if (b == 1) dma_x(c1, buf ^ 1, 0, 3);
+                if (b == 2) dma_x(c1, buf ^ 1, 3, 5);
                 const u32x4 raw = *reinterpret_cast<const u32x4 *>(wqs + (b * BN + 32 * wave + l32) * 16);
                 i32x4 aop;
                 aop.x = (int32_t)((raw.x >> shift) & 0x0f0f0f0fu);
@@ -279,13 +288,10 @@ __global__ __launch_bounds__(g2::kThreads, 2) void gemm_q4s_mfma_kernel(const ui
                 store_w(buf ^ 1);
                 __syncthreads();    // publishes stage c+1, retires the reads of buffer `buf`
                 zero_tail_headers(buf ^ 1);
-                if (c + 2 < n_stages) {
-                    dma_x(c + 2, buf);
-                    load_w(c + 2, buf);
-                }
             }
         }
 
+        JJO_GEMM_VMCNT(0);  // the last stage's repeated loads
         // ---- store: y[m][n] = 8 * acc ----
     #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
@@ -321,6 +327,8 @@ __global__ __launch_bounds__(g2::kThreads, 2) void gemm_q4s_mfma_kernel(const ui
 
 hipError_t launch_gemm_q4s_mfma(const void *w, const void *xq, float *y, int K, int N, int M, bool split,
                                 hipStream_t stream) {
+    // The row offsets inside a tile are 32 bits.
+    if (K >= kMaxTileK) return launch_gemm_mfma64(w, xq, y, K, N, M, stream, 64, split);
     const void *kern = split ? (const void *)gemm_q4s_mfma_kernel<true> : (const void *)gemm_q4s_mfma_kernel<false>;
     hipError_t e = ensure_dynamic_lds(kern, g2::kSmemBytes);
     if (e != hipSuccess) return e;

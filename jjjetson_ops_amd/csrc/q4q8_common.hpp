@@ -36,6 +36,10 @@ hipError_t ensure_dynamic_lds(const void *kernel, size_t bytes);
 // C ABI checked the device).
 int device_cu_count();
 
+// Row length up to which a tile's byte offsets (at most 128 rows of K/32*18 bytes) fit 32 bits;
+// longer rows take the kernels with 64-bit row addresses.
+constexpr int kMaxTileK = 1 << 25;
+
 // Kernel launchers (asynchronous on `stream`).  Shapes are validated by the
 // C-ABI layer before these are called.
 hipError_t launch_quantize_q8_1(const float *x, void *y, int64_t K, int64_t ne1, int64_t nz,
