@@ -89,7 +89,11 @@ __device__ __forceinline__ void kslice_offsets(uint32_t (&off)[3], int r0, int l
 // wave's own LDS; rows and tokens past the tile's end re-read the last valid one.
 // wq / wd: per row tile, the weight run (nibble plane when split) and the scale plane at
 // the tile's first row; woff: the lane's byte offsets below them (kslice_offsets).
-template <int RT, int CT, bool SPLIT>
+// SPREAD: the next stage's DMA goes out one instruction per block instead of in one burst,
+// where the waves' bursts queue for each other (64 x 64 tiles: 256 tokens N=4096 K=4096 18.4
+// -> 16.9 us, 512 tokens N=14336 96 -> 92.5).  Smaller tiles and the experts' short slices
+// need its earlier start more (E=8 top-2 FFN, 32 tokens: 225 us in a burst, 259 spread).
+template <int RT, int CT, bool SPLIT, bool SPREAD>
 __device__ __forceinline__ void kslice_loop(f32x16 (&acc)[RT][CT], uint8_t *stage, const uint8_t *const (&wq)[RT],
                                             const uint8_t *const (&wd)[RT], const uint32_t (&woff)[RT][3],
                                             const uint8_t *xb, size_t x_stride, uint32_t xlim, int s_beg, int s_end) {
@@ -99,6 +103,39 @@ __device__ __forceinline__ void kslice_loop(f32x16 (&acc)[RT][CT], uint8_t *stag
     float *wde = reinterpret_cast<float *>(stage + L::kOffScale);
     // Inline asm: the compiler would order every later LDS access behind these; their
     // completion is waited for at the top of a stage.
+    constexpr int kPieces = 3 * RT + L::kXRuns;
+    // One DMA instruction of a stage, for the spread form: the weights, which come from
+    // further away, first.
+    auto dma_piece = [&](int k, int s) {
+        if (k >= 3 * RT) {
+            const int i = k - 3 * RT;
+            const uint32_t m0v = __builtin_amdgcn_readfirstlane(stage_lds + i * 1024);
+            if ((i + 1) * 1024 <= L::kXBytes || lane < 32)
+                asm volatile("global_load_lds_dwordx4 %0, %1"
+                             :
+                             : "v"(min((uint32_t)(i * 1024 + lane * 16), xlim)), "s"(xb + (size_t)s * x_stride),
+                               "{m0}"(m0v)
+                             : "memory");
+            return;
+        }
+        const int rt = k / 3, i = k % 3;
+        const uint32_t m0v = __builtin_amdgcn_readfirstlane(stage_lds + L::kOffW + rt * L::kWTile + i * 1024);
+        if constexpr (!SPLIT)
+            asm volatile("global_load_lds_dwordx3 %0, %1"
+                         :
+                         : "v"(woff[rt][i]), "s"(wq[rt] + (size_t)s * (4 * kQ4BlockBytes)), "{m0}"(m0v)
+                         : "memory");
+        else if (i < 2)
+            asm volatile("global_load_lds_dwordx4 %0, %1"
+                         :
+                         : "v"(woff[rt][i]), "s"(wq[rt] + (size_t)s * 64), "{m0}"(m0v)
+                         : "memory");
+        else
+            asm volatile("global_load_lds_dword %0, %1"
+                         :
+                         : "v"(woff[rt][i]), "s"(wd[rt] + (size_t)s * 8), "{m0}"(m0v)
+                         : "memory");
+    };
     auto dma = [&](int s) {
         const uint8_t *px = xb + (size_t)s * x_stride;
 #pragma unroll
@@ -151,116 +188,23 @@ __device__ __forceinline__ void kslice_loop(f32x16 (&acc)[RT][CT], uint8_t *stag
     constexpr int kOrder[4] = {0, 2, 1, 3};
     constexpr int kJobs = 4 * RT * CT;  // 32x32 blocks of a stage
     if (s_beg < s_end) dma(s_beg);
-    for (int s = s_beg; s < s_end; ++s) {
-        JJO_GEMM_VMCNT(0);  // stage s has landed
-        asm volatile("" ::: "memory");
-        uint32_t raw[RT][9];
-        i32x4 xv[CT][4];
-        u32x4 hdr[CT];
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) {
-            const uint8_t *p = stage + L::kOffW + rt * L::kWTile;
-            if constexpr (SPLIT) {
-                const int sw = (l32 >> 2) & 3;
-                const u32x4 a = *reinterpret_cast<const u32x4 *>(p + l32 * 64 + 16 * ((2 * hh) ^ sw));
-                const u32x4 b = *reinterpret_cast<const u32x4 *>(p + l32 * 64 + 16 * ((2 * hh + 1) ^ sw));
-#pragma unroll
-                for (int k = 0; k < 4; ++k) { raw[rt][k] = a[k]; raw[rt][4 + k] = b[k]; }
-                raw[rt][8] = *reinterpret_cast<const uint32_t *>(p + 2048 + lane * 4);
-            } else {
-#pragma unroll
-                for (int i = 0; i < 3; ++i) {
-                    const u32x3 a = *reinterpret_cast<const u32x3 *>(p + (l32 * 6 + 3 * hh + i) * 16);
-#pragma unroll
-                    for (int k = 0; k < 3; ++k) raw[rt][3 * i + k] = a[k];
-                }
-            }
+    if constexpr (SPREAD) {
+        for (int s = s_beg; s < s_end - 1; ++s) {
+#define KSLICE_MORE true
+#include "gemm_kslice_stage.inc"
+#undef KSLICE_MORE
         }
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) {
-            const uint8_t *p = stage + (32 * ct + l32) * kQ8BlockBytes;
-            hdr[ct] = *reinterpret_cast<const u32x4 *>(p);
-#pragma unroll
-            for (int b = 0; b < 4; ++b) xv[ct][b] = *reinterpret_cast<const i32x4 *>(p + 16 + 32 * b + 16 * hh);
+        if (s_beg < s_end) {
+            const int s = s_end - 1;
+#define KSLICE_MORE false
+#include "gemm_kslice_stage.inc"
+#undef KSLICE_MORE
         }
-        asm volatile("" ::: "memory");
-        JJO_GEMM_LGKM0();  // stage s is in registers: its bytes may be overwritten
-        asm volatile("" ::: "memory");
-        if (s + 1 < s_end) dma(s + 1);
-
-        // ---- weights: nibbles -> int8 operands of the four blocks, scales/8 -> fp32 ----
-        uint32_t d16[RT];  // the lane's two fp16 scales: its K slots of the s_x MFMA
-        i32x4 aop[RT][4];
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) {
-            uint32_t q[2][4];
-            if constexpr (SPLIT) {
-                d16[rt] = raw[rt][8];
-#pragma unroll
-                for (int k = 0; k < 4; ++k) { q[0][k] = raw[rt][k]; q[1][k] = raw[rt][4 + k]; }
-            } else {
-                d16[rt] = (raw[rt][0] & 0xffffu) | (raw[rt][4] & 0xffff0000u);
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    q[0][k] = __builtin_amdgcn_alignbyte(raw[rt][k + 1], raw[rt][k], 2);
-                    q[1][k] = raw[rt][5 + k];
-                }
-            }
-            float *dst = wde + rt * 128 + 2 * hh * 32 + epi_perm(l32);
-            dst[0] = 0.125f * __half2float(__ushort_as_half((unsigned short)(d16[rt] & 0xffffu)));
-            dst[32] = 0.125f * __half2float(__ushort_as_half((unsigned short)(d16[rt] >> 16)));
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    // lanes 0-31 hold block i, lanes 32-63 block 2+i; after the swap the first
-                    // register is block i (low nibbles | high nibbles), the second block 2+i
-                    const auto r = __builtin_amdgcn_permlane32_swap(q[i][k] & 0x0f0f0f0fu,
-                                                                    (q[i][k] >> 4) & 0x0f0f0f0fu, false, false);
-                    aop[rt][i][k] = (int32_t)r[0];
-                    aop[rt][2 + i][k] = (int32_t)r[1];
-                }
-        }
-
-        // ---- 32x32 blocks: the MFMA of block j+1 runs under the epilogue of block j ----
-        i32x16 d[2];
-        float wv[16];
-        auto load_wv = [&](int g) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const f32x4 v = *reinterpret_cast<const f32x4 *>(wde + (g % RT) * 128 + kOrder[g / RT] * 32 + 16 * hh + 4 * i);
-#pragma unroll
-                for (int k = 0; k < 4; ++k) wv[4 * i + k] = v[k];
-            }
-        };
-        load_wv(0);
-        d[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(aop[0][kOrder[0]], xv[0][kOrder[0]], bias, 0, 0, 0);
-#pragma unroll
-        for (int j = 0; j < kJobs; ++j) {
-            const int rt = (j / CT) % RT, ct = j % CT, b = kOrder[j / (RT * CT)];
-            if (j + 1 < kJobs) {
-                const int rn = ((j + 1) / CT) % RT, cn = (j + 1) % CT, bn = kOrder[(j + 1) / (RT * CT)];
-                d[(j + 1) & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(aop[rn][bn], xv[cn][bn], bias, 0, 0, 0);
-            }
-            if (ct == 0 && j > 0) load_wv(j / CT);
-            float dx = __half2float(__ushort_as_half((unsigned short)(hdr[ct][b] & 0xffffu)));
-            asm("" : "+v"(dx));  // keep it fp32: no v_fma_mix in the epilogue
-            __builtin_amdgcn_sched_barrier(0);
-            epilogue_f32(acc[rt][ct], d[j & 1], wv, dx, dx * -kBias);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        // sum_b d_w * (-s_x) of the stage: lane half hh holds blocks 2*hh and 2*hh+1 in its
-        // first two K slots of both operands, zeros in the others.
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) {
-            const uint32_t h0 = hh ? hdr[ct][2] : hdr[ct][0], h1 = hh ? hdr[ct][3] : hdr[ct][1];
-            const u32x2 sx = {((h0 >> 16) | (h1 & 0xffff0000u)) ^ 0x80008000u, 0u};
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt) {
-                const u32x2 dw = {d16[rt], 0u};
-                acc[rt][ct] = __builtin_amdgcn_mfma_f32_32x32x8f16(
-                    __builtin_bit_cast(f16x4, dw), __builtin_bit_cast(f16x4, sx), acc[rt][ct], 0, 0, 0);
-            }
+    } else {
+        for (int s = s_beg; s < s_end; ++s) {
+#define KSLICE_MORE false
+#include "gemm_kslice_stage.inc"
+#undef KSLICE_MORE
         }
     }
 }
@@ -293,7 +237,7 @@ __global__ __launch_bounds__(64 * WK, WAVES_PER_SIMD) void gemm_kslice_kernel(
         wd[rt] = w + ((size_t)N * 16 + (size_t)n0 * 2) * nb;  // split: the scale plane
         kslice_offsets<SPLIT>(woff[rt], 32 * rt, N - 1 - n0, nb);
     }
-    kslice_loop<RT, CT, SPLIT>(acc, smem + wave * L::kWave, wq, wd, woff, xq + (size_t)m0 * kQ8BlockBytes,
+    kslice_loop<RT, CT, SPLIT, RT * CT == 4>(acc, smem + wave * L::kWave, wq, wd, woff, xq + (size_t)m0 * kQ8BlockBytes,
                                (size_t)M * kQ8BlockBytes, min(32 * CT, M - m0) * kQ8BlockBytes - 16,
                                (int)((int64_t)wave * nsb / WK), (int)((int64_t)(wave + 1) * nsb / WK));
 
@@ -413,7 +357,7 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_kslice_grouped_kernel(
         constexpr int C = decltype(ct_tag)::value;
         const int valid = min(32 * C, m_end - m0);
         f32x16 acc[RT][C];
-        kslice_loop<RT, C, SPLIT>(acc, smem + wave * KsliceLds<RT, C, SPLIT>::kWave, wq, wd, woff, xb, x_stride,
+        kslice_loop<RT, C, SPLIT, false>(acc, smem + wave * KsliceLds<RT, C, SPLIT>::kWave, wq, wd, woff, xb, x_stride,
                                   valid * kQ8BlockBytes - 16, s_beg, s_end);
         __syncthreads();  // every wave is done with its staging area
         constexpr int kTile = C * 256, kItems = RT * kTile;
