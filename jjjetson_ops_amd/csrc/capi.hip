@@ -1084,14 +1084,9 @@ int moe_ffn_run(bool split, void *stream, const float *x, const float *logits, c
             if ((e = launch_moe_route_decode(x, logits, T, H, E, top_k, ws.route_w, ws.ids, ws.offsets,
                                              ws.src_route, ws.dst_of_route, ws.xp, s)) != hipSuccess)
                 return hip_fail(e, "moe_ffn routing");
-        } else {  // more routes (top_k > 24) than the one-launch routing holds: four launches
-            if ((e = launch_quantize_q8_1(x, ws.xq, H, T, 1, s)) != hipSuccess) return hip_fail(e, "moe_ffn quantize x");
-            if ((e = launch_moe_top_k(logits, ws.route_w, ws.ids, T, E, top_k, s)) != hipSuccess)
-                return hip_fail(e, "moe_ffn top_k");
-            if ((e = launch_moe_dispatch(ws.ids, R, E, ws.offsets, ws.src_route, ws.dst_of_route, s)) != hipSuccess)
-                return hip_fail(e, "moe_ffn dispatch");
-            if ((e = launch_moe_gather_q8_1(ws.xq, ws.src_route, ws.xp, T, R, top_k, H, s)) != hipSuccess)
-                return hip_fail(e, "moe_ffn gather");
+        } else if ((e = launch_moe_route(x, logits, T, H, E, top_k, ws.route_w, ws.ids, ws.offsets, ws.src_route,
+                                         ws.dst_of_route, ws.xp, s)) != hipSuccess) {
+            return hip_fail(e, "moe_ffn routing");  // more routes (top_k > 24) than the one-launch routing holds
         }
         const int per_expert = mean_routes(R, E);
         if ((e = launch_gemv_routed(w_gate, w_up, ws.xp, ws.offsets, E, R, per_expert, ws.gate_up, 2 * I, H, I,
@@ -1106,19 +1101,15 @@ int moe_ffn_run(bool split, void *stream, const float *x, const float *logits, c
             return hip_fail(e, "moe_ffn combine");
         return JJO_OK;
     }
-    // 1) x -> Q8_1 (once per token), 2) top-k gating, 3) stable dispatch + Q8_1 row gather
-    if ((e = launch_quantize_q8_1(x, ws.xq, H, T, 1, s)) != hipSuccess) return hip_fail(e, "moe_ffn quantize x");
-    if ((e = launch_moe_top_k(logits, ws.route_w, ws.ids, T, E, top_k, s)) != hipSuccess)
-        return hip_fail(e, "moe_ffn top_k");
-    if ((e = launch_moe_dispatch(ws.ids, R, E, ws.offsets, ws.src_route, ws.dst_of_route, s)) != hipSuccess)
-        return hip_fail(e, "moe_ffn dispatch");
-    if ((e = launch_moe_gather_q8_1(ws.xq, ws.src_route, ws.xp, T, R, top_k, H, s)) != hipSuccess)
-        return hip_fail(e, "moe_ffn gather");
-    // 4) gate|up of every route's expert in one grouped launch whose epilogue applies
+    // 1) top-k gating, 2) stable dispatch, x -> Q8_1 (once per token) at its routes' rows
+    if ((e = launch_moe_route(x, logits, T, H, E, top_k, ws.route_w, ws.ids, ws.offsets, ws.src_route,
+                              ws.dst_of_route, ws.xp, s)) != hipSuccess)
+        return hip_fail(e, "moe_ffn routing");
+    // 3) gate|up of every route's expert in one grouped launch whose epilogue applies
     //    SwiGLU and writes the Q8_1 input of the down projection (no fp32 gate|up)
     if ((e = run_gate_up_swiglu(w_gate, w_up, ws.xp, ws.offsets, E, ws.midq, H, I, R, split, s)) != hipSuccess)
         return hip_fail(e, "moe_ffn gate_up_swiglu");
-    // 5) down projection, 6) weighted combine back to token order
+    // 4) down projection, 5) weighted combine back to token order
     if ((e = run_grouped(w_down, nullptr, 0, ws.midq, ws.offsets, E, nullptr, ws.eout, I, H, R, split, s)) !=
         hipSuccess)
         return hip_fail(e, "moe_ffn down");

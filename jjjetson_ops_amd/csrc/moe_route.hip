@@ -23,64 +23,113 @@ namespace {
 // value first and takes a later e only when strictly greater; ids[k] in selection
 // order.  That keeps the smallest id of the largest non-NaN value, or expert 0 when
 // v(0) is NaN (nothing compares greater than NaN), and it re-selects a taken expert
-// once only -inf values are left; the wave computes exactly that: each lane holds
-// experts lane + 64j in registers with a taken bit each, and a lane-local best
-// (value, id) over its non-NaN values is reduced over the wave (larger value, then
-// smaller id).
+// once only -inf values are left; the wave computes exactly that.  Each lane holds
+// experts lane + 64j as unsigned keys in the order of the values (-0 as +0; NaN and
+// experts past the end 0, below the key of -inf; a taken expert becomes -inf): a
+// round is a lane-local maximum, a DPP maximum over the wave and one ballot of the
+// lanes that hold it, whose smallest (j, lane) is the smallest id.  The rounds are a
+// serial chain, so their latency is the kernel's time: shuffles of (value, id, valid)
+// over 16 registers a lane took 11.9 us for 100 tokens, 64 experts, top-6; PER =
+// ceil(num_experts / 64) keys and DPP take 4.8 us.
 // Weights: softmax over the selected logits (delayed_softmax, moe_top_k.cu:12-55,
 // 190-195): max = the first selected value, e_i = expf(v_i - max), and the sum is
 // the 32-lane xor butterfly of warp_reduce_xor_sum (include/cuda_utils.cuh:37-43)
 // over e_0..e_{top_k-1} held by lanes 0..top_k-1 (zeros elsewhere), run on the
 // lanes themselves, so the association order is the reference's; w_i = e_i * (1 / sum).
-constexpr int kTopKPerLane = 16;  // 1024 experts / 64 lanes
+__device__ __forceinline__ uint64_t ballot64(bool p) { return __ballot(p); }
+
+constexpr uint32_t kNegInfKey = 0x007fffffu;  // order_key(-inf)
+
+// Unsigned key in the order of the non-NaN floats, -0 equal to +0; NaN gives 0.
+__device__ __forceinline__ uint32_t order_key(float x) {
+    const uint32_t u = __float_as_uint(x + 0.0f);  // -0 + 0 = +0
+    return x == x ? u ^ (uint32_t)(((int32_t)u >> 31) | (int32_t)0x80000000) : 0u;
+}
+
+__device__ __forceinline__ float order_value(uint32_t k) {
+    return __uint_as_float(k & 0x80000000u ? k ^ 0x80000000u : ~k);
+}
+
+// Maximum / sum of the wave's 64 values, in every lane: row shifts inside the rows of
+// 16, then row_bcast15 and row_bcast31; a lane without a source takes 0.
+#define JJO_WAVE_FOLD(v, OP)                                                          \
+    v = OP(v, (decltype(v))__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false)); \
+    v = OP(v, (decltype(v))__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false)); \
+    v = OP(v, (decltype(v))__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false)); \
+    v = OP(v, (decltype(v))__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false)); \
+    v = OP(v, (decltype(v))__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false)); \
+    v = OP(v, (decltype(v))__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false))
+
+__device__ __forceinline__ uint32_t umax32(uint32_t a, uint32_t b) { return a > b ? a : b; }
+__device__ __forceinline__ uint32_t uadd32(uint32_t a, uint32_t b) { return a + b; }
+
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
+    JJO_WAVE_FOLD(v, umax32);
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+__device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
+    JJO_WAVE_FOLD(v, uadd32);
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+#undef JJO_WAVE_FOLD
 
 // All 64 lanes of the wave call this for one token; lanes 0..top_k-1 write
-// weights[lane] and ids[lane].
+// weights[lane] and ids[lane].  num_experts <= 64 * PER.
+template <int PER>
 __device__ __forceinline__ void top_k_token(const float *__restrict__ row, int num_experts, int top_k,
                                             float *__restrict__ weights, int *__restrict__ ids, int lane) {
-    float v[kTopKPerLane];
+    uint32_t key[PER];
+    float v0 = 0.0f;
 #pragma unroll
-    for (int j = 0; j < kTopKPerLane; ++j) {
+    for (int j = 0; j < PER; ++j) {
         const int e = lane + 64 * j;
-        v[j] = e < num_experts ? row[e] : 0.0f;
+        const float x = e < num_experts ? row[e] : 0.0f;
+        if (j == 0) v0 = x;
+        key[j] = e < num_experts ? order_key(x) : 0u;
     }
-    const float v0 = __shfl(v[0], 0);  // expert 0's logit
-    uint32_t taken = 0;                // bit j: expert lane + 64j
-    bool taken0 = false;
+    v0 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v0)));  // expert 0's logit
+    bool nan0 = v0 != v0;  // until expert 0 is taken (and -inf)
     float my_v = 0.0f, mx = 0.0f;
     int my_id = 0;
     for (int k = 0; k < top_k; ++k) {
-        float bv = -INFINITY;
-        int bid = 0x7fffffff;
-        bool ok = false;
+        uint32_t bk = key[0];
+        int bj = 0;
 #pragma unroll
-        for (int j = 0; j < kTopKPerLane; ++j) {
-            const int e = lane + 64 * j;
-            const float x = ((taken >> j) & 1u) ? -INFINITY : v[j];
-            if (e < num_experts && x == x && (!ok || x > bv)) {  // ids ascend with j
-                bv = x;
-                bid = e;
-                ok = true;
+        for (int j = 1; j < PER; ++j)
+            if (key[j] > bk) {  // ids ascend with j
+                bk = key[j];
+                bj = j;
             }
-        }
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            const float ov = __shfl_xor(bv, off);
-            const int oid = __shfl_xor(bid, off);
-            const bool ook = __shfl_xor((int)ok, off) != 0;
-            if (ook && (!ok || ov > bv || (ov == bv && oid < bid))) {
-                bv = ov;
-                bid = oid;
-                ok = true;
-            }
-        }
-        const float v0k = taken0 ? -INFINITY : v0;
-        if (v0k != v0k) {  // v(0) NaN: the scan never leaves expert 0
-            bv = v0k;
+        float bv;
+        int bid;
+        if (nan0) {  // v(0) NaN: the scan never leaves expert 0
+            bv = v0;
             bid = 0;
+            nan0 = false;
+        } else {  // expert 0 is a candidate: the maximum is at least the key of -inf
+            const uint32_t m = wave_max(bk);
+            uint64_t tied = ballot64(bk == m);
+            int j = 0;
+            if constexpr (PER > 1) {
+                if ((tied & (tied - 1)) == 0) {
+                    j = __builtin_amdgcn_readlane(bj, __builtin_ctzll(tied));
+                } else {
+                    for (j = 0; j < PER - 1; ++j) {
+                        const uint64_t at_j = ballot64(bk == m && bj == j);
+                        if (at_j != 0) {
+                            tied = at_j;
+                            break;
+                        }
+                    }
+                }
+            }
+            bid = 64 * j + __builtin_ctzll(tied);
+            bv = order_value(m);
         }
-        if (lane == (bid & 63)) taken |= 1u << (bid >> 6);
-        taken0 |= bid == 0;
+#pragma unroll
+        for (int j = 0; j < PER; ++j)
+            if (lane + 64 * j == bid) key[j] = kNegInfKey;
         if (k == 0) mx = bv;
         if (lane == k) {
             my_v = bv;
@@ -100,14 +149,15 @@ __device__ __forceinline__ void top_k_token(const float *__restrict__ row, int n
 
 constexpr int kTopKWaves = 4;  // tokens per workgroup
 
+template <int PER>
 __global__ __launch_bounds__(64 * kTopKWaves) void moe_top_k_kernel(const float *__restrict__ logits,
                                                                     float *__restrict__ weights,
                                                                     int *__restrict__ ids, int num_tokens,
                                                                     int num_experts, int top_k) {
     const int t = blockIdx.x * kTopKWaves + (threadIdx.x >> 6);
     if (t >= num_tokens) return;  // whole waves
-    top_k_token(logits + (size_t)t * num_experts, num_experts, top_k, weights + (size_t)t * top_k,
-                ids + (size_t)t * top_k, threadIdx.x & 63);
+    top_k_token<PER>(logits + (size_t)t * num_experts, num_experts, top_k, weights + (size_t)t * top_k,
+                     ids + (size_t)t * top_k, threadIdx.x & 63);
 }
 
 // ---------------------------------------------------------------- dispatch
@@ -116,9 +166,10 @@ __global__ __launch_bounds__(64 * kTopKWaves) void moe_top_k_kernel(const float 
 // (a stable sort by expert, as cub::DeviceRadixSort::SortPairs over the arange in
 // moe_dispatch_sota.cu:127-136), and expert_offsets[e] = #{routes with expert < e}
 // (the lower-bound search of moe_dispatch_sota.cu:45-71).
+// One workgroup, a serial chain of steps.  A step's ranks come from one ballot per
+// bit of the expert id (lanes whose ids agree in every bit), not one round per
+// distinct expert: 600 routes over 64 experts 10.0 us -> 3.4 us.
 constexpr int kDispatchWaves = 16;
-
-__device__ __forceinline__ uint64_t ballot64(bool p) { return __ballot(p); }
 
 __global__ __launch_bounds__(64 * kDispatchWaves) void moe_dispatch_kernel(
     const int *__restrict__ ids, int num_routes, int num_experts, int32_t *__restrict__ expert_offsets,
@@ -143,9 +194,13 @@ __global__ __launch_bounds__(64 * kDispatchWaves) void moe_dispatch_kernel(
     // expert's base, then its waves' bases follow in wave order.
     __shared__ int wave_sum[kDispatchWaves];
     const int e_own = threadIdx.x;
+    int c_own[kDispatchWaves];
     int tot = 0;
-    if (e_own < num_experts)
-        for (int w = 0; w < kDispatchWaves; ++w) tot += cnt[w * num_experts + e_own];
+#pragma unroll
+    for (int w = 0; w < kDispatchWaves; ++w) {
+        c_own[w] = e_own < num_experts ? cnt[w * num_experts + e_own] : 0;
+        tot += c_own[w];
+    }
     int incl = tot;  // inclusive scan within the wave
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -158,31 +213,29 @@ __global__ __launch_bounds__(64 * kDispatchWaves) void moe_dispatch_kernel(
     for (int w = 0; w < wave; ++w) base += wave_sum[w];
     if (e_own < num_experts) {
         expert_offsets[e_own] = base;
+#pragma unroll
         for (int w = 0; w < kDispatchWaves; ++w) {
-            const int c = cnt[w * num_experts + e_own];
             cnt[w * num_experts + e_own] = base;
-            base += c;
+            base += c_own[w];
         }
         if (e_own == num_experts - 1) expert_offsets[num_experts] = base;
     }
     __syncthreads();
     // stable placement: 64 routes per step in route order; lanes with equal experts
-    // are ranked by lane index through a ballot per distinct expert of the step
+    // are ranked by lane index
+    const int id_bits = 32 - __builtin_clz(num_experts);
     for (int r0 = r_beg; r0 < r_end; r0 += 64) {
         const int r = r0 + lane;
         const bool live = r < r_end;
-        const int e = live ? min(max(ids[r], 0), num_experts - 1) : -1;
-        uint64_t todo = ballot64(live);
-        int pos = 0;
-        while (todo != 0) {
-            const int leader = __builtin_ctzll(todo);
-            const int el = __shfl(e, leader);
-            const uint64_t grp = ballot64(live && e == el);
-            if (e == el && live) pos = my[el] + __builtin_popcountll(grp & ((1ull << lane) - 1ull));
-            if (lane == leader) my[el] += __builtin_popcountll(grp);
-            todo &= ~grp;
+        const int e = live ? min(max(ids[r], 0), num_experts - 1) : 0;
+        uint64_t grp = ballot64(live);
+        for (int b = 0; b < id_bits; ++b) {
+            const uint64_t one = ballot64((e >> b) & 1);
+            grp &= (e >> b) & 1 ? one : ~one;
         }
         if (live) {
+            const int pos = my[e] + __builtin_popcountll(grp & ((1ull << lane) - 1ull));
+            if (lane == 63 - __builtin_clzll(grp)) my[e] = pos + 1;  // after every lane's read: one wave
             src_route[pos] = r;
             dst_of_route[r] = pos;
         }
@@ -228,6 +281,7 @@ __device__ __forceinline__ void quantize_store_q8_1(float4 v, int i0, uint8_t *_
     if ((iqs & 31) == 0) *reinterpret_cast<uint32_t *>(out + 4 * (iqs / 32)) = ds;
 }
 
+template <int PER>
 __global__ __launch_bounds__(256) void moe_route_decode_kernel(
     const float *__restrict__ x, const float *__restrict__ logits, int num_tokens, int hidden, int num_experts,
     int top_k, float *__restrict__ route_w, int *__restrict__ ids, int32_t *__restrict__ expert_offsets,
@@ -249,8 +303,8 @@ __global__ __launch_bounds__(256) void moe_route_decode_kernel(
     }
     // 2) top-k of every token, one wave per token
     for (int t = threadIdx.x >> 6; t < num_tokens; t += blockDim.x >> 6)
-        top_k_token(logits + (size_t)t * num_experts, num_experts, top_k, s_w + t * top_k, s_ids + t * top_k,
-                    threadIdx.x & 63);
+        top_k_token<PER>(logits + (size_t)t * num_experts, num_experts, top_k, s_w + t * top_k, s_ids + t * top_k,
+                         threadIdx.x & 63);
     __syncthreads();
     // 3) stable positions (ids clamped to a valid expert, as in moe_dispatch_kernel)
     for (int r = threadIdx.x; r < R; r += blockDim.x) {
@@ -287,6 +341,117 @@ __global__ __launch_bounds__(256) void moe_route_decode_kernel(
         quantize_store_q8_1(*reinterpret_cast<const float4 *>(row + i0), i0, xp, R, pos);
 }
 
+// ---------------------------------------------------------------- routing of larger batches
+// After the top-k, one launch for the rest of the routing: workgroup t + 1 loads up to
+// 4096 values of token t's row, finds the positions of its top_k routes and stores the
+// row's Q8_1 blocks (quantize_group8: the quantizer's bytes) at each of them.
+// SORT (up to kRouteSortMax routes): a position is the number of routes whose
+// (expert, route) is smaller, counted over all ids by each workgroup (16 compares a
+// thread and route at most), and workgroup 0 writes the expert offsets; otherwise
+// moe_dispatch_kernel has written the tables.  Bound by latency: the separate
+// quantizer, dispatch and gather took 4.7 + 10.0 + 4.8 us and two launches more for
+// 100 tokens x 2048, top-6 of 64; this one 7.5 us.
+constexpr int kRouteSortMax = 4096;
+
+template <bool SORT>
+__global__ __launch_bounds__(256) void moe_route_quantize_kernel(
+    const float *__restrict__ x, const int *__restrict__ ids, int num_tokens, int hidden, int num_experts, int top_k,
+    int32_t *__restrict__ expert_offsets, int32_t *__restrict__ src_route, int32_t *__restrict__ dst_of_route,
+    uint8_t *__restrict__ xp) {
+    constexpr int kIds = SORT ? kRouteSortMax / 256 : 1;
+    __shared__ int s_cnt[SORT ? 1024 : 1];  // routes of each expert (num_experts <= 1024)
+    __shared__ int s_part[4][32];           // top_k <= 32
+    __shared__ int s_pos[32];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int R = num_tokens * top_k;
+    if (blockIdx.x == 0) {
+        if constexpr (SORT) {
+            if (blockIdx.y != 0) return;
+            for (int e = tid; e < 1024; e += 256) s_cnt[e] = 0;
+            __syncthreads();
+            for (int r = tid; r < R; r += 256) atomicAdd(&s_cnt[min(max(ids[r], 0), num_experts - 1)], 1);
+            __syncthreads();
+            int c[4], tot = 0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) tot += c[i] = s_cnt[4 * tid + i];
+            int incl = tot;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const int o = __shfl_up(incl, d);
+                if (lane >= d) incl += o;
+            }
+            if (lane == 63) s_part[wave][0] = incl;
+            __syncthreads();
+            int base = incl - tot;
+            for (int w = 0; w < wave; ++w) base += s_part[w][0];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (4 * tid + i <= num_experts) expert_offsets[4 * tid + i] = base;
+                base += c[i];
+            }
+            if (tid == 255 && num_experts == 1024) expert_offsets[1024] = base;
+        }
+        return;
+    }
+    const int t = blockIdx.x - 1;
+    const int col0 = blockIdx.y * (1024 * kDecodeRowRegs);
+    // 1) the row in flight (hidden % 128 == 0: every 32-lane half-wave is live or idle as a whole)
+    const float *row = x + (size_t)t * hidden;
+    float4 xv[kDecodeRowRegs];
+#pragma unroll
+    for (int i = 0; i < kDecodeRowRegs; ++i) {
+        const int i0 = col0 + (tid + i * 256) * 4;
+        xv[i] = i0 < hidden ? *reinterpret_cast<const float4 *>(row + i0) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    // 2) the positions of the token's routes
+    if constexpr (SORT) {
+        int id[kIds];  // expert * 4096 + route
+#pragma unroll
+        for (int i = 0; i < kIds; ++i) {
+            const int r = tid + 256 * i;
+            id[i] = r < R ? min(max(ids[r], 0), num_experts - 1) * kRouteSortMax + r : 0x7fffffff;
+        }
+        const int r_own = t * top_k + min(lane, top_k - 1);  // lane k: route k of the token
+        const int own_id = min(max(ids[r_own], 0), num_experts - 1) * kRouteSortMax + r_own;
+        for (int k = 0; k < top_k; ++k) {
+            const int own = __builtin_amdgcn_readlane(own_id, k);
+            uint32_t n = 0;
+#pragma unroll
+            for (int i = 0; i < kIds; ++i) n += id[i] < own;
+            n = wave_sum(n);
+            if (lane == 0) s_part[wave][k] = (int)n;
+        }
+        __syncthreads();
+        if (tid < top_k) {
+            const int pos = s_part[0][tid] + s_part[1][tid] + s_part[2][tid] + s_part[3][tid];
+            s_pos[tid] = pos;
+            if (blockIdx.y == 0) {
+                dst_of_route[t * top_k + tid] = pos;
+                src_route[pos] = t * top_k + tid;
+            }
+        }
+    } else {
+        if (tid < top_k) s_pos[tid] = dst_of_route[t * top_k + tid];
+    }
+    __syncthreads();
+    // 3) quantize once, store at every position
+#pragma unroll
+    for (int i = 0; i < kDecodeRowRegs; ++i) {
+        const int i0 = col0 + (tid + i * 256) * 4;
+        if (i0 < hidden) {
+            uint32_t ds;
+            const uint32_t q = quantize_group8(xv[i].x, xv[i].y, xv[i].z, xv[i].w, &ds);
+            uint8_t *base = xp + (size_t)(i0 / kQSuper) * R * kQ8BlockBytes;
+            const int iqs = i0 % kQSuper;
+            for (int k = 0; k < top_k; ++k) {
+                uint8_t *out = base + (size_t)s_pos[k] * kQ8BlockBytes;
+                *reinterpret_cast<uint32_t *>(out + 16 + iqs) = q;
+                if ((iqs & 31) == 0) *reinterpret_cast<uint32_t *>(out + 4 * (iqs / 32)) = ds;
+            }
+        }
+    }
+}
+
 // ---------------------------------------------------------------- combine
 // y[t][h] = sum over k in order of w[t,k] * expert_out[dst(t,k)][h], acc from 0
 // (moe_combine_sota.cu:21-41).  Four consecutive h per thread.
@@ -312,10 +477,19 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const float *__restric
 
 }  // namespace
 
+// KERNEL<PER> with PER keys a lane for num_experts <= 64 * PER.
+#define JJO_BY_EXPERTS(KERNEL, grid, block, ...)                                                      \
+    do {                                                                                              \
+        if (num_experts <= 64) hipLaunchKernelGGL(KERNEL<1>, grid, block, 0, stream, __VA_ARGS__);         \
+        else if (num_experts <= 128) hipLaunchKernelGGL(KERNEL<2>, grid, block, 0, stream, __VA_ARGS__);   \
+        else if (num_experts <= 256) hipLaunchKernelGGL(KERNEL<4>, grid, block, 0, stream, __VA_ARGS__);   \
+        else hipLaunchKernelGGL(KERNEL<16>, grid, block, 0, stream, __VA_ARGS__);                          \
+    } while (0)
+
 hipError_t launch_moe_top_k(const float *logits, float *weights, int *ids, int num_tokens, int num_experts,
                             int top_k, hipStream_t stream) {
-    hipLaunchKernelGGL(moe_top_k_kernel, dim3((num_tokens + kTopKWaves - 1) / kTopKWaves), dim3(64 * kTopKWaves), 0,
-                       stream, logits, weights, ids, num_tokens, num_experts, top_k);
+    const dim3 grid((num_tokens + kTopKWaves - 1) / kTopKWaves), block(64 * kTopKWaves);
+    JJO_BY_EXPERTS(moe_top_k_kernel, grid, block, logits, weights, ids, num_tokens, num_experts, top_k);
     return hipGetLastError();
 }
 
@@ -340,9 +514,29 @@ hipError_t launch_moe_route_decode(const float *x, const float *logits, int num_
                                   int top_k, float *route_w, int *ids, int32_t *expert_offsets, int32_t *src_route,
                                   int32_t *dst_of_route, void *xp, hipStream_t stream) {
     if (num_tokens * top_k > kMoeDecodeRoutes || hidden % kQSuper != 0) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(moe_route_decode_kernel, dim3((unsigned)(num_tokens * top_k)), dim3(256), 0, stream, x,
-                       logits, num_tokens, hidden, num_experts, top_k, route_w, ids, expert_offsets, src_route,
-                       dst_of_route, (uint8_t *)xp);
+    JJO_BY_EXPERTS(moe_route_decode_kernel, dim3((unsigned)(num_tokens * top_k)), dim3(256), x, logits, num_tokens,
+                   hidden, num_experts, top_k, route_w, ids, expert_offsets, src_route, dst_of_route, (uint8_t *)xp);
+    return hipGetLastError();
+}
+
+hipError_t launch_moe_route(const float *x, const float *logits, int num_tokens, int hidden, int num_experts,
+                            int top_k, float *route_w, int *ids, int32_t *expert_offsets, int32_t *src_route,
+                            int32_t *dst_of_route, void *xp, hipStream_t stream) {
+    if (hidden % kQSuper != 0 || num_experts > 1024 || top_k > 32) return hipErrorInvalidValue;
+    hipError_t e = launch_moe_top_k(logits, route_w, ids, num_tokens, num_experts, top_k, stream);
+    if (e != hipSuccess) return e;
+    const int R = num_tokens * top_k;
+    const int cols = 1024 * kDecodeRowRegs;
+    const dim3 grid((unsigned)num_tokens + 1, (unsigned)((hidden + cols - 1) / cols));
+    if (R <= kRouteSortMax) {
+        hipLaunchKernelGGL(moe_route_quantize_kernel<true>, grid, dim3(256), 0, stream, x, ids, num_tokens, hidden,
+                           num_experts, top_k, expert_offsets, src_route, dst_of_route, (uint8_t *)xp);
+        return hipGetLastError();
+    }
+    if ((e = launch_moe_dispatch(ids, R, num_experts, expert_offsets, src_route, dst_of_route, stream)) != hipSuccess)
+        return e;
+    hipLaunchKernelGGL(moe_route_quantize_kernel<false>, grid, dim3(256), 0, stream, x, ids, num_tokens, hidden,
+                       num_experts, top_k, expert_offsets, src_route, dst_of_route, (uint8_t *)xp);
     return hipGetLastError();
 }
 

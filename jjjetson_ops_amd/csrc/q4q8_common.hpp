@@ -132,6 +132,10 @@ constexpr int kMoeDecodeRoutes = 384;
 hipError_t launch_moe_route_decode(const float *x, const float *logits, int num_tokens, int hidden, int num_experts,
                                   int top_k, float *route_w, int *ids, int32_t *expert_offsets, int32_t *src_route,
                                   int32_t *dst_of_route, void *xp, hipStream_t stream);
+// The same routing (the same tables and bytes) for any batch, in two or three launches.
+hipError_t launch_moe_route(const float *x, const float *logits, int num_tokens, int hidden, int num_experts,
+                            int top_k, float *route_w, int *ids, int32_t *expert_offsets, int32_t *src_route,
+                            int32_t *dst_of_route, void *xp, hipStream_t stream);
 hipError_t launch_moe_combine(const float *expert_out, const int32_t *dst_of_route, const float *route_weights,
                               float *y, int num_tokens, int hidden, int top_k, hipStream_t stream);
 // fp32 -> Q4_0 over a flat run of n_blocks 32-value blocks.
