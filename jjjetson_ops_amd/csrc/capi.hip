@@ -565,8 +565,7 @@ namespace {
 #endif
 constexpr int kGroupedGemvRoutes = JJO_GROUPED_GEMV_ROUTES;
 bool grouped_gemv(int n_routes, int K) { return n_routes <= kGroupedGemvRoutes && K <= kGemvMaxK; }
-// Routes per active expert expected.  The grouped entries, which do not know their
-// tokens, take it as the routed GEMV's chunk.
+// Routes per active expert expected: the chunk size of the routed GEMV.
 int mean_routes(int n_routes, int n_experts) {
     const int active = n_experts < n_routes ? n_experts : n_routes;
     return (n_routes + active - 1) / active;
@@ -619,8 +618,7 @@ int mat_mul_q4_0_q8_1_grouped_device(const void *d_w_q4_0, const void *d_x_q8_1,
     if ((rc = require_gfx950()) != JJO_OK) return rc;
     hipError_t e = grouped_gemv(n_routes, ncols_k)
                        ? launch_gemv_routed(d_w_q4_0, nullptr, d_x_q8_1, d_expert_offsets, n_experts, n_routes,
-                                            mean_routes(n_routes, n_experts), mean_routes(n_routes, n_experts),
-                                            d_y, nrows_out, ncols_k, nrows_out,
+                                            mean_routes(n_routes, n_experts), d_y, nrows_out, ncols_k, nrows_out,
                                             false, (hipStream_t)stream, d_route_dst)
                        : run_grouped(d_w_q4_0, nullptr, 0, d_x_q8_1, d_expert_offsets, n_experts, d_route_dst, d_y,
                                      ncols_k, nrows_out, n_routes, false, (hipStream_t)stream);
@@ -641,8 +639,7 @@ int mat_mul_q4_0s_q8_1_grouped_device(const void *d_w_split, const void *d_x_q8_
     if ((rc = require_gfx950()) != JJO_OK) return rc;
     hipError_t e = grouped_gemv(n_routes, ncols_k)
                        ? launch_gemv_routed(d_w_split, nullptr, d_x_q8_1, d_expert_offsets, n_experts, n_routes,
-                                            mean_routes(n_routes, n_experts), mean_routes(n_routes, n_experts),
-                                            d_y, nrows_out, ncols_k, nrows_out,
+                                            mean_routes(n_routes, n_experts), d_y, nrows_out, ncols_k, nrows_out,
                                             true, (hipStream_t)stream, d_route_dst)
                        : run_grouped(d_w_split, nullptr, 0, d_x_q8_1, d_expert_offsets, n_experts, d_route_dst, d_y,
                                      ncols_k, nrows_out, n_routes, true, (hipStream_t)stream);
@@ -1005,8 +1002,7 @@ int moe_q4_0_gate_up_device(void *stream, const void *w_gate, const void *w_up, 
     hipError_t e =
         grouped_gemv(n_routes, hidden_size)
             ? launch_gemv_routed(w_gate, w_up, x_q8_1_permuted, expert_offsets, num_experts, n_routes,
-                                 mean_routes(n_routes, num_experts), mean_routes(n_routes, num_experts),
-                                 gate_up, 2 * intermediate_size, hidden_size,
+                                 mean_routes(n_routes, num_experts), gate_up, 2 * intermediate_size, hidden_size,
                                  intermediate_size, false, (hipStream_t)stream)
             : run_grouped(w_gate, w_up, intermediate_size, x_q8_1_permuted, expert_offsets, num_experts, nullptr,
                           gate_up, hidden_size, 2 * intermediate_size, n_routes, false, (hipStream_t)stream);
@@ -1080,8 +1076,8 @@ int moe_ffn_run(bool split, void *stream, const float *x, const float *logits, c
     const int R = T * top_k;
     hipError_t e;
     if (moe_decode_path(T, H, I, E, top_k)) {
-        // Chunk size of the routed GEMVs: from the mean routes per active expert and the
-        // most (a token's experts are distinct: T).
+        // Chunk size of the routed GEMVs: the mean routes per active expert (an expert
+        // with more takes several chunks with its weights held in registers).
         // 1) quantize + top-k + dispatch + gather, 2) gate|up (both matrices, one
         // launch) -> fp32 [R][2I], 3) SwiGLU + Q8_1, 4) down projection, 5) combine
         if (R <= kMoeDecodeRoutes) {
@@ -1093,12 +1089,12 @@ int moe_ffn_run(bool split, void *stream, const float *x, const float *logits, c
             return hip_fail(e, "moe_ffn routing");  // more routes (top_k > 24) than the one-launch routing holds
         }
         const int per_expert = mean_routes(R, E);
-        if ((e = launch_gemv_routed(w_gate, w_up, ws.xp, ws.offsets, E, R, per_expert, T, ws.gate_up, 2 * I, H, I,
+        if ((e = launch_gemv_routed(w_gate, w_up, ws.xp, ws.offsets, E, R, per_expert, ws.gate_up, 2 * I, H, I,
                                     split, s)) != hipSuccess)
             return hip_fail(e, "moe_ffn gate_up (routed GEMV)");
         if ((e = launch_swiglu_quantize_q8_1(ws.gate_up, ws.midq, nullptr, I, R, s)) != hipSuccess)
             return hip_fail(e, "moe_ffn swiglu");
-        if ((e = launch_gemv_routed(w_down, nullptr, ws.midq, ws.offsets, E, R, per_expert, T, ws.eout, H, I, H, split,
+        if ((e = launch_gemv_routed(w_down, nullptr, ws.midq, ws.offsets, E, R, per_expert, ws.eout, H, I, H, split,
                                     s)) != hipSuccess)
             return hip_fail(e, "moe_ffn down (routed GEMV)");
         if ((e = launch_moe_combine(ws.eout, ws.dst_of_route, ws.route_w, y, T, H, top_k, s)) != hipSuccess)

@@ -1168,6 +1168,9 @@ hipError_t launch_gemv_q4s_fused(const void *w, const float *x, void *xq_out, fl
     return launch_m<true, 1, JJO_Q4S_U1F, true>(w, x, (uint8_t *)xq_out, y, K, N, stream);
 }
 
+#ifndef JJO_RT_MT4_MAXK_SPLIT
+#define JJO_RT_MT4_MAXK_SPLIT 16384
+#endif
 // Rows per wave of the one-route routed instances: split as the dense decode
 // kernel; block_q4_0 at 4 instead of 2 (E=8 top-2 FFN T=4: 142.9 -> 138.7 us; split
 // at 2 or 8 and block_q4_0 at 1 were slower).
@@ -1192,26 +1195,17 @@ hipError_t launch_gemv_q4s_fused(const void *w, const float *x, void *xq_out, fl
 #ifndef JJO_RT_U4_BLOCK
 #define JJO_RT_U4_BLOCK kU4
 #endif
-// An expert with more routes than the chunk re-requests its weights and re-stages
-// activations for every further chunk, so the chunk is twice the mean where a second
-// chunk is likely (a router over 8 experts gives 38% of its active experts two routes
-// or more at a mean of one), never more than an expert can hold.  Split, one box, us
-// per FFN, E=8 top-2 4096 x 14336, chunk = mean -> this: T=2 70.0 -> 51.0 (4 routes:
-// 56.5), T=4 124.3 -> 100.1 (109.7), T=6 133.6 -> 120.4, T=8 179.6 -> 172.7; E=64 top-6
-// 2048 x 1408, T=8 57.3 -> 46.9.  A single token stays at one route (42.5; two: 45.7).
-// block_q4_0 rows past one K slice keep two routes at a mean of two: their 4-route
-// instances hold fewer waves (T=8 183.9; four: 194.0).
-int gemv_routed_chunk(int mean_routes, int most_routes, int K, bool split) {
-    const int want = mean_routes <= 1 || (mean_routes == 2 && !split && K > 4096) ? 2 : 4;
-    const int most = most_routes <= 1 ? 1 : most_routes <= 2 ? 2 : 4;
-    return want < most ? want : most;
+int gemv_routed_chunk(int max_routes_per_expert, int K, bool split) {
+    const int cap = split && K > JJO_RT_MT4_MAXK_SPLIT ? 2 : 4;
+    const int mt = max_routes_per_expert <= 1 ? 1 : max_routes_per_expert <= 2 ? 2 : 4;
+    return mt < cap ? mt : cap;
 }
 
 hipError_t launch_gemv_routed(const void *w, const void *w2, const void *xq, const int32_t *expert_offsets,
-                              int n_experts, int n_routes, int mean_routes, int most_routes, float *y, int ldy, int K, int N,
+                              int n_experts, int n_routes, int max_routes_per_expert, float *y, int ldy, int K, int N,
                               bool split, hipStream_t stream, const int32_t *route_dst) {
-    if (K > 16384 || most_routes < 1) return hipErrorInvalidValue;
-    const int mt = gemv_routed_chunk(mean_routes, most_routes, K, split);
+    if (K > 16384 || max_routes_per_expert < 1) return hipErrorInvalidValue;
+    const int mt = gemv_routed_chunk(max_routes_per_expert, K, split);
     const int slots = n_experts < n_routes ? n_experts : n_routes;
     const RouteArgs ra{expert_offsets, (const uint8_t *)w2, route_dst, n_experts, n_routes, slots, ldy};
     const int gy = slots * (w2 != nullptr ? 2 : 1);
