@@ -292,6 +292,17 @@ __device__ __forceinline__ void finish_f32(uint8_t *xs, uint8_t *__restrict__ xq
 // (each chunk re-stages only activation rows), so every weight byte of an active
 // expert is read once whatever its route count.  Output row p (a sorted route
 // position) starts at y + p * ldy, or at y + route_dst[p] * ldy.
+// M = 1 (a mean of at most one route per active expert): a slot is one route instead,
+// and the workgroups that read the same rows for an expert's routes are 8 apart in the
+// grid (blockIdx.x = 8 * slot + row group % 8, blockIdx.y = row group / 8, blockIdx.z =
+// which): the same XCD at the same time, so the later ones read its L2.  A second pass
+// of one workgroup re-read the rows after they had left the cache and lengthened the
+// grid's tail: E=8 top-2 4096 x 14336, random routing, FFN us (block_q4_0 / split), T=2
+// 67.0 / 69.7 -> 49.1 / 55.8, T=4 125.1 / 124.3 -> 108.6 / 103.4; one route on every expert
+// 143 / 125, unchanged; E=64 top-6 2048 x 1408, T=8 60.6 / 57.5 -> 50.2 / 47.3 (48 experts
+// of one route each: 57.0 / 53.3 -> 58.6 / 54.1).  Chunks of two routes were as fast with
+// random routing but hold 6 waves per SIMD instead of 8: 10-14% slower with one route on
+// every expert.
 struct RouteArgs {
     const int32_t *offsets;    // [n_experts + 1]
     const uint8_t *w2;         // second stacked matrix, or null
@@ -315,10 +326,31 @@ __device__ __forceinline__ void expert_range(const RouteArgs &ra, int e, int &be
 }
 
 // false: this workgroup has no routes (the same for all its waves).
+template <bool BY_ROUTE>
 __device__ __forceinline__ bool route_tile(const RouteArgs &ra, int mt, RouteTile &t) {
-    const int which = (int)blockIdx.y >= ra.slots;
-    int slot = (int)blockIdx.y - which * ra.slots;
+    const int which = BY_ROUTE ? (int)blockIdx.z : (int)blockIdx.y >= ra.slots;
+    int slot = BY_ROUTE ? (int)(blockIdx.x >> 3) : (int)blockIdx.y - which * ra.slots;
     const int lane = threadIdx.x & 63;
+    if constexpr (BY_ROUTE) {
+        for (int e0 = 0; e0 < ra.n_experts; e0 += 64) {
+            bool holds = false;
+            if (e0 + lane < ra.n_experts) {
+                int b, en;
+                expert_range(ra, e0 + lane, b, en);
+                holds = b <= slot && slot < en;
+            }
+            const uint64_t bal = __ballot(holds);
+            if (bal != 0) {
+                t.expert = e0 + __builtin_ctzll(bal);
+                t.which = which;
+                t.m0 = slot;
+                t.mc = 1;
+                t.end = slot + 1;
+                return true;
+            }
+        }
+        return false;
+    }
     int e = -1;
     for (int e0 = 0; e0 < ra.n_experts; e0 += 64) {
         bool nonempty = false;
@@ -401,12 +433,15 @@ __global__ __launch_bounds__(64 * JS * RG) void gemv_q4_0_q8_1_kernel(const uint
     const int hrow = R2 ? (lane >> 5) * U : 0;         // R2: lanes 32..63 on rows U further
     const bool live = p < P;
     const size_t row_bytes = (size_t)nb * kQ4BlockBytes;
-    const int r0 = (blockIdx.x * RG + rg) * kRowsW;
+    constexpr bool kByRoute = ROUTED && M == 1;
+    const int bx = kByRoute ? (int)(8 * blockIdx.y + (blockIdx.x & 7)) : (int)blockIdx.x;
+    if (kByRoute && bx * RG * kRowsW >= N) return;
+    const int r0 = (bx * RG + rg) * kRowsW;
     const int n_items = FUSED ? 2 * nb : M * nb;
     const int rounds = (n_items + kThreadsWG - 1) / kThreadsWG;
     RouteTile rt{0, 0, 0, M, M};
     if constexpr (ROUTED) {
-        if (!route_tile(ra, M, rt)) return;
+        if (!route_tile<kByRoute>(ra, M, rt)) return;
         w = (rt.which ? ra.w2 : w) + (size_t)rt.expert * N * row_bytes;
         y += (size_t)rt.which * N;
     }
@@ -467,7 +502,7 @@ __global__ __launch_bounds__(64 * JS * RG) void gemv_q4_0_q8_1_kernel(const uint
         const int rg = ROUTED ? (tid >> 6) / JS : rg_o;
         const int p = ROUTED ? (R2 ? (lane & 31) : lane + 64 * js) : p_o;
         const bool live = p < P;
-        const int r0 = ROUTED ? (int)(blockIdx.x * RG + rg) * kRowsW : r0_o;
+        const int r0 = ROUTED ? (bx * RG + rg) * kRowsW : r0_o;
         // 3) activation planes of the whole K range in LDS, once per workgroup (routed:
         //    per chunk of routes)
         for (int r = (ROUTED && again) ? 0 : EARLY; r < rounds; ++r) {  // the rest, load-then-use
@@ -613,7 +648,7 @@ __global__ __launch_bounds__(64 * JS * RG) void gemv_q4_0_q8_1_kernel(const uint
                     }
             }
         }
-        if constexpr (!ROUTED) {
+        if constexpr (!ROUTED || kByRoute) {
             break;
         } else {
             // the expert's next chunk of routes: the same weight rows, new activation rows
@@ -622,10 +657,9 @@ __global__ __launch_bounds__(64 * JS * RG) void gemv_q4_0_q8_1_kernel(const uint
             mcc = min(M, rt.end - m0c);
             again = true;
             __syncthreads();  // every wave is done with the records and partial sums
-            if constexpr (M <= 2) {
+            if constexpr (M == 2) {
                 // Re-request the weight rows (L2) rather than keep them live through
-                // the pass: held, they cost the 1- and 2-route kernels half their
-                // occupancy, for a loop that only a tie-broken top-k repeat reaches.
+                // the pass: held, they cost the 2-route kernel half its occupancy.
                 const int pl = min(p, P - 1);
                 for (int u = 0; u < U; ++u)
                     load_pair(wb[u], w + (size_t)min(r0 + (R2 ? (lane >> 5) * U : 0) + u, N - 1) * row_bytes +
@@ -748,13 +782,16 @@ __global__ __launch_bounds__(64 * JS * RG) void gemv_q4s_kernel(const uint8_t *_
     const int bk0 = 128 * js + lane;       // this lane's two blocks
     const int bk1 = bk0 + 64;
     const int c0 = min(bk0, nb - 1), c1 = min(bk1, nb - 1);
-    const int r0 = (blockIdx.x * RG + rg) * kRowsW;
+    constexpr bool kByRoute = ROUTED && M == 1;
+    const int bx = kByRoute ? (int)(8 * blockIdx.y + (blockIdx.x & 7)) : (int)blockIdx.x;
+    if (kByRoute && bx * RG * kRowsW >= N) return;
+    const int r0 = (bx * RG + rg) * kRowsW;
     const int n_items = FUSED ? 2 * nb : M * nb;
     const int rounds = (n_items + kThreadsWG - 1) / kThreadsWG;
     RouteTile rt{0, 0, 0, M, M};
     size_t plane_rows = N, row0 = 0;  // rows of the buffer's planes, first row of this matrix
     if constexpr (ROUTED) {
-        if (!route_tile(ra, M, rt)) return;
+        if (!route_tile<kByRoute>(ra, M, rt)) return;
         if (rt.which) w = ra.w2;
         plane_rows = (size_t)ra.n_experts * N;
         row0 = (size_t)rt.expert * N;
@@ -817,7 +854,7 @@ __global__ __launch_bounds__(64 * JS * RG) void gemv_q4s_kernel(const uint8_t *_
         const int bk0 = ROUTED ? 128 * js + lane : bk0_o;
         const int bk1 = bk0 + 64;
         const int c0 = min(bk0, nb - 1), c1 = min(bk1, nb - 1);
-        const int r0 = ROUTED ? (int)(blockIdx.x * RG + rg) * kRowsW : r0_o;
+        const int r0 = ROUTED ? (bx * RG + rg) * kRowsW : r0_o;
         // 3) activation records of the whole K range in LDS, once per workgroup (routed:
         //    per chunk of routes)
         for (int r = (ROUTED && again) ? 0 : EARLY; r < rounds; ++r) {  // the rest, load-then-use
@@ -933,7 +970,7 @@ __global__ __launch_bounds__(64 * JS * RG) void gemv_q4s_kernel(const uint8_t *_
                     }
             }
         }
-        if constexpr (!ROUTED) {
+        if constexpr (!ROUTED || kByRoute) {
             break;
         } else {
             // the expert's next chunk of routes: the same weight rows, new activation rows
@@ -942,7 +979,7 @@ __global__ __launch_bounds__(64 * JS * RG) void gemv_q4s_kernel(const uint8_t *_
             mcc = min(M, rt.end - m0c);
             again = true;
             __syncthreads();  // every wave is done with the records and partial sums
-            if constexpr (M <= 2) {  // (as in gemv_q4_0_q8_1_kernel)
+            if constexpr (M == 2) {  // (as in gemv_q4_0_q8_1_kernel)
                 for (int u = 0; u < U; ++u) {
                     const size_t base = (row0 + (size_t)min(r0 + u, N - 1)) * nb;
                     const size_t base1 = R2 ? (row0 + (size_t)min(r0 + U + u, N - 1)) * nb : base;
@@ -1059,6 +1096,7 @@ hipError_t launch_cfg(const void *w, const void *xin, uint8_t *xq_out, float *y,
     constexpr int kRowsW = R2 ? 2 * U : U;
     const int groups = (N + kRowsW - 1) / kRowsW;
     const int blocks = (groups + RG - 1) / RG;
+    const dim3 grid = ROUTED && M == 1 ? dim3(8 * ra.slots, (blocks + 7) / 8, gy / ra.slots) : dim3(blocks, gy);
     const size_t smem = SPLIT ? ((size_t)M * (K / 32) + 1) * kRecS : ((size_t)M * (K / 64) + 1) * kRec;
     const void *kern = SPLIT ? (const void *)gemv_q4s_kernel<M, U, JS, RG, FUSED, EARLY, ROUTED, R2>
                              : (const void *)gemv_q4_0_q8_1_kernel<M, U, JS, RG, FUSED, EARLY, ROUTED, R2>;
@@ -1068,10 +1106,10 @@ hipError_t launch_cfg(const void *w, const void *xin, uint8_t *xq_out, float *y,
         if (e != hipSuccess) return e;
     }
     if constexpr (SPLIT) {
-        hipLaunchKernelGGL((gemv_q4s_kernel<M, U, JS, RG, FUSED, EARLY, ROUTED, R2>), dim3(blocks, gy),
+        hipLaunchKernelGGL((gemv_q4s_kernel<M, U, JS, RG, FUSED, EARLY, ROUTED, R2>), grid,
                            dim3(64 * JS * RG), smem, stream, (const uint8_t *)w, xin, xq_out, y, K, N, ra);
     } else {
-        hipLaunchKernelGGL((gemv_q4_0_q8_1_kernel<M, U, JS, RG, FUSED, EARLY, ROUTED, R2>), dim3(blocks, gy),
+        hipLaunchKernelGGL((gemv_q4_0_q8_1_kernel<M, U, JS, RG, FUSED, EARLY, ROUTED, R2>), grid,
                            dim3(64 * JS * RG), smem, stream, (const uint8_t *)w, xin, xq_out, y, K, N, ra);
     }
     return hipGetLastError();
@@ -1205,8 +1243,9 @@ hipError_t launch_gemv_routed(const void *w, const void *w2, const void *xq, con
                               int n_experts, int n_routes, int max_routes_per_expert, float *y, int ldy, int K, int N,
                               bool split, hipStream_t stream, const int32_t *route_dst) {
     if (K > 16384 || max_routes_per_expert < 1) return hipErrorInvalidValue;
-    const int mt = gemv_routed_chunk(max_routes_per_expert, K, split);
-    const int slots = n_experts < n_routes ? n_experts : n_routes;
+    int mt = gemv_routed_chunk(max_routes_per_expert, K, split);
+    if (mt == 1 && N >= 1 << 20) mt = 2;  // the by-route grid's y limit
+    const int slots = mt == 1 || n_routes < n_experts ? n_routes : n_experts;
     const RouteArgs ra{expert_offsets, (const uint8_t *)w2, route_dst, n_experts, n_routes, slots, ldy};
     const int gy = slots * (w2 != nullptr ? 2 : 1);
     if (split) {

@@ -58,7 +58,8 @@ hipError_t launch_gemv_q4s_fused(const void *w, const float *x, void *xq_out, fl
 // Routed GEMV over E stacked [N][K] experts (MoE decode): routes sorted by expert,
 // expert_offsets[E+1], Q8_1 route rows superblock-major over n_routes rows; each
 // active expert's weights are read once, its routes taken in chunks sized for
-// max_routes_per_expert (routes per active expert expected; more take more chunks).
+// max_routes_per_expert (routes per active expert expected; more take more chunks; at one,
+// a workgroup takes one route and an expert's workgroups share its rows through L2).
 // Sorted route p's output row starts at y + p * ldy, or at y + route_dst[p] * ldy
 // (route_dst nullable, entries unchecked).  w2 (nullable): a second stacked matrix of the same shape,
 // computed in the same launch into columns N..2N-1 of each output row.  K <= 16384;
