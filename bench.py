@@ -221,7 +221,7 @@ def time_moe(dev, steps, warmup):
 def time_moe_ffn(dev, steps, warmup, split=False, T=512):
     """The whole Q4_0 MoE FFN of the same layer shape (8 experts, top-2, T tokens,
     H=4096, I=14336): quantize, top-k, dispatch, gate|up, SwiGLU+quantize, down,
-    combine -- seven launches per step at T=512 (gate|up, SwiGLU and its Q8_1
+    combine -- five launches per step at T=512 (gate|up, SwiGLU and its Q8_1
     quantization are one); five at decode sizes (T <= 16: one routing launch, routed
     GEMVs).  Decode steps read only their active experts (2 x 99 MB at T=1), which
     the 256 MB MALL could keep between steps: there the step rotates over 4 router
@@ -274,7 +274,7 @@ def time_moe_ffn(dev, steps, warmup, split=False, T=512):
 
     for i in range(warmup):
         step(i)
-    launches = 5 if decode else 7
+    launches = 5
     avg = _time_steps(step, steps, launches) / steps
     R = T * topk
     ops = 2.0 * R * 3 * I * H

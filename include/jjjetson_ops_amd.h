@@ -362,10 +362,11 @@ int moe_combine_device(void *stream, const float *expert_out, const int32_t *dst
 /*
  * The whole Q4_0 MoE FFN on device pointers: x fp32 [T][H], logits fp32 [T][E],
  * y fp32 [T][H].  `workspace` (256-byte aligned) holds every intermediate; its
- * size is moe_q4_0_ffn_workspace_bytes(...).  Seven launches (quantize x, top-k,
- * dispatch, gather, gate|up with SwiGLU and Q8_1, down, combine); at 16 tokens or
- * fewer, or at most two routes per active expert on average (H, I <= 16384), five
- * (routing in one launch -- four above 384 routes --, gate|up over the active experts
+ * size is moe_q4_0_ffn_workspace_bytes(...).  Five launches (top-k,
+ * dispatch with x -> Q8_1 at its routes' rows -- a launch more above 4096 routes --,
+ * gate|up with SwiGLU and Q8_1, down, combine); at 16 tokens or fewer, or at most two
+ * routes per active expert on average (H, I <= 16384), five as well (routing in one
+ * launch -- two above 384 routes --, gate|up over the active experts
  * into an fp32 [R][2I] part of the workspace, SwiGLU + Q8_1, down, combine).  No
  * allocation, asynchronous on `stream`.  H % 128 == 0, I % 128 == 0.
  */
