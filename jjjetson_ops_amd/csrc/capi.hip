@@ -183,8 +183,8 @@ int small_tile_rows(int N, int M) {
 // K=2048..11008, N=2048..14336, 48..2048 tokens; 32-row tiles: 0.36 + 0.0007 us per
 // workgroup; 64: 0.24 + 0.00157; 128 x 128: 3.03 us per round of two workgroups per CU).
 // Measured, tiled against K-sliced (us): N=4096, K=4096: 48 tokens 21.6 / 8.4, 100: 22.3 /
-// 11.8, 512: 37.4 / 31.1, 2048: 105-110 / 112 (stays tiled); K=11008: 48: 52 / 18, 1024:
-// 157-167 / 140; N=14336, K=4096: 100: 37.6 / 31, 512: 105-117 / 98, 1024: 197 / 197.
+// 11.8, 512: 37.4 / 30.1, 2048: 105-110 / 112 (stays tiled); K=11008: 48: 52 / 18, 1024:
+// 157-167 / 140; N=14336, K=4096: 100: 37.6 / 30.4, 512: 105-117 / 96, 1024: 197 / 197.
 int kslice_shape(int K, int N, int M) {
     if (M > 65535 || K >= kMaxTileK) return -1;
     const double stages = K / kQSuper, cus = device_cus();
