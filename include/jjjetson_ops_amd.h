@@ -185,6 +185,21 @@ int mat_mul_q4_0_q8_1_block_sums_device(const void *d_w_q4_0, const void *d_x_q8
                                         void *stream);
 
 /*
+ * DIAGNOSTIC ONLY (for tests and crossover tuning; no counterpart in the reference).
+ * jjo_mm_auto_kernel: the kernel that the matmul entries run for a shape with 16-byte
+ * aligned weights (split != 0: in the split layout), a JJO_ALGO_* value or
+ * JJO_KERNEL_KSLICE plus a tile form: 0: 32 rows x 32 tokens, 1: 32 x 64, 2: 64 x 64, each on
+ * eight waves, 3: 64 x 64 on four; -1 for an invalid shape.  Launches nothing (256 CUs
+ * are assumed before a device has been used).
+ * jjo_mm_kernel_device: the matmul on that kernel, in either layout: JJO_ALGO_MFMA64,
+ * JJO_ALGO_MFMA32, JJO_ALGO_MFMA_W32 or a JJO_KERNEL_KSLICE form.
+ */
+#define JJO_KERNEL_KSLICE 16
+int jjo_mm_auto_kernel(int ncols_k, int nrows_out, int batch, int split);
+int jjo_mm_kernel_device(const void *d_w, const void *d_x_q8_1, float *d_y, int ncols_k, int nrows_out,
+                         int batch, int split, int kernel, void *stream);
+
+/*
  * DIAGNOSTIC ONLY (a measurement probe, not part of the drop-in path; no
  * counterpart in the reference): one plain coalesced read of `bytes`
  * (a multiple of 16) from d_src, the HBM read floor of a single launch that the

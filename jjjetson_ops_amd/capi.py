@@ -26,6 +26,7 @@ ALGO_SKINNY_LDS = 4
 ALGO_MFMA64 = 5
 ALGO_MFMA32 = 6
 ALGO_MFMA_W32 = 7
+KERNEL_KSLICE = 16  # + tile form 0..3 (mm_auto_kernel, mm_kernel)
 
 QK = 32
 QSUPER = 128
@@ -47,6 +48,8 @@ EXPORTED_SYMBOLS = (
     "mat_mul_q4_0_q8_1_block_sums_device",
     "mat_mul_q4_0_q8_1_grouped_device",
     "mat_mul_q4_0s_q8_1_grouped_device",
+    "jjo_mm_auto_kernel",
+    "jjo_mm_kernel_device",
     "jjo_read_floor_device",
     "linear_q4_0_workspace_bytes",
     "linear_q4_0_forward_device",
@@ -141,6 +144,10 @@ def lib() -> ctypes.CDLL:
         L.mat_mul_q4_0_q8_1_grouped_device.argtypes = [vp, vp, vp, i32, vp, vp, i32, i32, i32, vp]
         L.mat_mul_q4_0s_q8_1_grouped_device.restype = i32
         L.mat_mul_q4_0s_q8_1_grouped_device.argtypes = [vp, vp, vp, i32, vp, vp, i32, i32, i32, vp]
+        L.jjo_mm_auto_kernel.restype = i32
+        L.jjo_mm_auto_kernel.argtypes = [i32, i32, i32, i32]
+        L.jjo_mm_kernel_device.restype = i32
+        L.jjo_mm_kernel_device.argtypes = [vp, vp, vp, i32, i32, i32, i32, i32, vp]
         L.jjo_read_floor_device.restype = i32
         L.jjo_read_floor_device.argtypes = [vp, i64, vp, vp]
         L.linear_q4_0_workspace_bytes.restype = i64
@@ -399,6 +406,30 @@ def grouped_mat_mul(w, xq, expert_offsets, y, K: int, N: int, n_routes: int, rou
     fn = lib().mat_mul_q4_0s_q8_1_grouped_device if split else lib().mat_mul_q4_0_q8_1_grouped_device
     _check(fn(_dev(w, "w"), _dev(xq, "xq"), _dev(expert_offsets, "offsets"), n_experts, rd, _dev(y, "y"), K, N,
               n_routes, _stream(stream)), "grouped_mat_mul")
+
+
+def mm_auto_kernel(K: int, N: int, M: int, split: bool = False) -> int:
+    """jjo_mm_auto_kernel: the kernel the matmul entries run for this shape (ALGO_* or
+    KERNEL_KSLICE + tile form)."""
+    k = int(lib().jjo_mm_auto_kernel(K, N, M, int(split)))
+    if k < 0:
+        _check(JJO_ERR_INVALID_ARG, "jjo_mm_auto_kernel")
+    return k
+
+
+def mm_kernel(w, xq, y, K: int, N: int, M: int, kernel: int, split: bool = False, stream=None) -> None:
+    """jjo_mm_kernel_device: mat_mul / mat_mul_split on a chosen tiled or K-sliced kernel."""
+    import torch
+    if y.dtype != torch.float32:
+        raise ValueError("y must be float32")
+    if w.numel() * w.element_size() < N * (K // QK) * Q4_BLOCK_BYTES:
+        raise ValueError("weight buffer too small")
+    if xq.numel() * xq.element_size() < M * (K // QSUPER) * Q8_BLOCK_BYTES:
+        raise ValueError("Q8_1 buffer too small")
+    if y.numel() < M * N:
+        raise ValueError("output buffer too small")
+    _check(lib().jjo_mm_kernel_device(_dev(w, "w"), _dev(xq, "xq"), _dev(y, "y"), K, N, M, int(split), kernel,
+                                      _stream(stream)), "jjo_mm_kernel_device")
 
 
 def read_floor(src, nbytes: int, out, stream=None) -> None:

@@ -178,27 +178,57 @@ int small_tile_rows(int N, int M) {
     return 2 * (int64_t)((N + 63) / 64) * ((M + 63) / 64) <= 3 * cus ? 32 : 64;
 }
 
-// The K-sliced mid-batch kernel's tile shape where it is estimated to beat the tiled GEMMs,
-// else -1.  Their time is a fixed part per 128-value stage plus one per workgroup (fitted to
-// K=2048..11008, N=2048..14336, 48..2048 tokens; 32-row tiles: 0.36 + 0.0007 us per
-// workgroup; 64: 0.24 + 0.00157; 128 x 128: 3.03 us per round of two workgroups per CU).
-// Measured, tiled against K-sliced (us): N=4096, K=4096: 48 tokens 21.6 / 8.4, 100: 22.3 /
-// 11.8, 512: 37.4 / 30.1, 2048: 105-110 / 112 (stays tiled); K=11008: 48: 52 / 18, 1024:
-// 157-167 / 140; N=14336, K=4096: 100: 37.6 / 30.4, 512: 105-117 / 96, 1024: 197 / 197.
-int kslice_shape(int K, int N, int M) {
-    if (M > 65535 || K >= kMaxTileK) return -1;
-    const double stages = K / kQSuper, cus = device_cus();
-    double tiled;
-    if (const int tr = small_tile_rows(N, M); tr != 0) {
-        const double wgs = (double)((N + tr - 1) / tr) * ((M + 63) / 64);
-        tiled = 4.0 + stages * (tr == 32 ? 0.36 + 0.0007 * wgs : 0.24 + 0.00157 * wgs);
-    } else {
-        const double tiles = (double)((N + 127) / 128) * ((M + 127) / 128);
-        tiled = 5.0 + stages * 3.03 * (tiles / (2.0 * cus) + 0.1);
+// Estimated time (us) of the tiled GEMM that small_tile_rows chooses, per layout (the split
+// 128 x 128 kernel is the faster one): 32-row tiles, 64 x 64 tiles (two rounds' worth per CU
+// overlap; a last round of at most one workgroup per CU is cheaper), 128 x 128 tiles in rounds
+// of two workgroups per CU, a last round that fills at most half of them at half the work.
+// Fitted with kShapes (gemm_kslice.hip) and as accurate.
+double tiled_us(int K, int N, int M, bool split) {
+    const int64_t cus = device_cus(), slots = 2 * cus;
+    const double stages = K / kQSuper;
+    const int tr = small_tile_rows(N, M);
+    if (tr == 32) {
+        const double wgs = (double)((N + 31) / 32) * ((M + 63) / 64);
+        return split ? 2.91 + stages * (0.540 + 0.000635 * wgs) : 3.08 + stages * (0.681 + 0.000510 * wgs);
     }
+    if (tr == 64) {
+        const int64_t g = (int64_t)((N + 63) / 64) * ((M + 63) / 64), rem = g % slots;
+        const double fixed = split ? 2.75 : 2.28, round = split ? 1.05 : 1.32;
+        const double full = round + (split ? 0.888 : 0.902) * stages, alone = round + (split ? 0.522 : 0.512) * stages;
+        return fixed + (double)(g / slots) * full + (rem == 0 ? 0.0 : rem > cus ? full : alone);
+    }
+    const int64_t g = (int64_t)((N + 127) / 128) * ((M + 127) / 128), rem = g % slots;
+    const int64_t halved = g < slots ? g : 2 * rem <= slots ? rem : 0;  // tiles run as two halves
+    const double round = 3.96, fixed = split ? 0.376 : 0.0;
+    return fixed + (double)((g - halved + slots - 1) / slots) * (round + (split ? 2.71 : 2.82) * stages) +
+           (double)((2 * halved + slots - 1) / slots) * (round + (split ? 1.60 : 1.47) * stages);
+}
+
+// A K-sliced tile shape runs a problem: 32-bit offsets inside a tile, tokens of one superblock.
+bool kslice_accepts(int shape, int K, int N, int M) {
+    return shape >= 0 && shape <= 3 && M <= 65535 && K < kMaxTileK;
+}
+
+// The K-sliced mid-batch kernel's tile shape where it is estimated to beat the tiled GEMMs,
+// else -1.  Measured, tiled against the best K-sliced shape (block_q4_0 / split, us): N=4096,
+// K=4096: 48 tokens 21.9 / 21.2 against 8.6 / 8.2, 512: 33.5 / 32.7 against 27.7 / 27.1, 1536: 85.2
+// / 82.8 against 76.1 / 75.1, 2048: 96.1 / 93.0 against 103 / 101 (stays tiled); K=11008, 1024
+// tokens: 151 / 147 against 128 / 127; N=14336, K=4096: 1024: 191 / 176 against 172 / 169, 2048:
+// 353 / 341 against 377 / 375.  Over the shapes fitted (11 000) the choice is 0.7% from the
+// best kernel on average and slower than the tiled GEMM by more than 5% for 0.4% of them (most at N=34000..58000 and up to
+// 64 tokens, just above a full round of workgroups).
+//   Short rows (K < 1536) with over 2^20 outputs stay tiled: eight waves have a stage or none
+// each and the outputs are what is left (K=768, N=11008, 129 tokens: 11.1 / 10.9 against 12.6 /
+// 12.1; K=1024, N=20480, 80: 14.4 / 14.0 against 15.6 / 15.2).  So do batches above 3072 tokens,
+// whose activation outgrows an XCD's L2 when every row tile walks all of it (K=1024, N=1024,
+// 4096 tokens: 18.6 / 18.0 against 22.1 / 21.8); from 1024 on, where a wrong choice costs
+// more than a right one gains, the estimate has to be 4% lower.
+int kslice_shape(int K, int N, int M, bool split) {
+    if (M > 3072 || (K < 1536 && (int64_t)N * M > 1 << 20)) return -1;
     double sliced;
     const int shape = kslice_pick(K, N, M, &sliced);
-    return sliced < 1.08 * tiled ? shape : -1;  // the fit reads 5-10% low
+    const double bar = (M > 1024 ? 0.96 : 1.0) * tiled_us(K, N, M, split);
+    return sliced < bar && kslice_accepts(shape, K, N, M) ? shape : -1;
 }
 
 int run_kslice(const void *w, const void *xq, float *y, int K, int N, int M, bool split, int shape, hipStream_t s) {
@@ -206,32 +236,32 @@ int run_kslice(const void *w, const void *xq, float *y, int K, int N, int M, boo
     return e == hipSuccess ? JJO_OK : hip_fail(e, "gemm_kslice launch");
 }
 
+// The kernel AUTO runs for a matmul in either layout: a JJO_ALGO_* value (MFMA_W32 is the
+// split layout's 128 x 128 kernel) or JJO_KERNEL_KSLICE + tile shape.
+//   The GEMV wins up to batch 4 on rows of one K-slice (K <= 4096); with more slices its
+// per-token cost grows and the skinny kernel wins from batch 3.  At K <= 4096 the LDS-resident
+// skinny kernel is 4-30% faster than the per-wave one from batch 5 (N=14336: 11.2-11.6 against
+// 12.0-14.0 us; N=11008: 9.0-9.4 against 11.5-13.4 us); at larger K the per-wave kernel is
+// faster.  Above batch 16 the K-sliced GEMM replaces both (24 tokens, N=14336, K=4096: 25.1 ->
+// 16.2 us; N=4096, K=11008: 27.6 -> 18.5 us) where it is faster than the tiled GEMMs; of
+// those the small tiles run while 128 x 128 tiles would not fill the chip well.
+int auto_kernel(const void *w, const void *xq, int K, int N, int M, bool split) {
+    const int64_t gemv_lds = (int64_t)M * (split ? (K / kQK) * 48 : (K / 64) * 80);
+    const bool gemv_ok = M <= kGemvMaxBatch && K <= kGemvMaxK && gemv_lds <= 150 * 1024;
+    if (gemv_ok && M <= (K <= 4096 ? kGemvPreferredBatch : 2)) return JJO_ALGO_GEMV;
+    if (K <= 4096 && M >= 5 && gemm_skinny_persist_supported(w, xq, K, M)) return JJO_ALGO_SKINNY_LDS;
+    if (M <= 16 && gemm_skinny_supported(w, xq, K, M)) return JJO_ALGO_SKINNY;
+    if (gemv_ok) return JJO_ALGO_GEMV;
+    if (const int shape = kslice_shape(K, N, M, split); shape >= 0) return JJO_KERNEL_KSLICE + shape;
+    if (gemm_skinny_supported(w, xq, K, M)) return JJO_ALGO_SKINNY;
+    if (const int tr = small_tile_rows(N, M); tr != 0) return tr == 32 ? JJO_ALGO_MFMA32 : JJO_ALGO_MFMA64;
+    return split ? JJO_ALGO_MFMA_W32 : JJO_ALGO_MFMA;
+}
+
 int run_mm(const void *w, const void *xq, float *y, int K, int N, int M, int algo, hipStream_t s) {
     if (algo == JJO_ALGO_AUTO) {
-        const bool gemv_ok = M <= kGemvMaxBatch && K <= kGemvMaxK && (int64_t)M * (K / 64) * 80 <= 150 * 1024;
-        // The GEMV wins up to batch 4 on rows of one K-slice (K <= 4096); with more
-        // slices its per-token cost grows and the skinny kernel wins from batch 3.
-        // Above batch 16 the K-sliced GEMM replaces both skinny kernels (24 tokens, N=14336,
-        // K=4096: 25.1 -> 16.2 us; N=4096, K=11008: 27.6 -> 18.5 us).
-        // At K <= 4096 the LDS-resident skinny kernel is 4-30% faster than the
-        // per-wave one from batch 5 (N=14336: 11.2-11.6 against 12.0-14.0 us; N=11008:
-        // 9.0-9.4 against 11.5-13.4 us); at larger K the per-wave kernel is faster.
-        if (gemv_ok && M <= (K <= 4096 ? kGemvPreferredBatch : 2))
-            algo = JJO_ALGO_GEMV;
-        else if (K <= 4096 && M >= 5 && gemm_skinny_persist_supported(w, xq, K, M))
-            algo = JJO_ALGO_SKINNY_LDS;
-        else if (M <= 16 && gemm_skinny_supported(w, xq, K, M))
-            algo = JJO_ALGO_SKINNY;
-        else if (gemv_ok)
-            algo = JJO_ALGO_GEMV;
-        else if (const int shape = kslice_shape(K, N, M); shape >= 0)
-            return run_kslice(w, xq, y, K, N, M, false, shape, s);
-        else if (gemm_skinny_supported(w, xq, K, M))
-            algo = JJO_ALGO_SKINNY;
-        else if (const int tr = small_tile_rows(N, M); tr != 0)
-            algo = tr == 32 ? JJO_ALGO_MFMA32 : JJO_ALGO_MFMA64;
-        else
-            algo = JJO_ALGO_MFMA;
+        algo = auto_kernel(w, xq, K, N, M, false);
+        if (algo >= JJO_KERNEL_KSLICE) return run_kslice(w, xq, y, K, N, M, false, algo - JJO_KERNEL_KSLICE, s);
     }
     hipError_t e;
     if (algo == JJO_ALGO_GEMV) {
@@ -453,41 +483,28 @@ int q4_0_to_split_device(const void *d_w_q4_0, void *d_w_split, int nrows, int n
 
 namespace {
 // Split-layout matmul from Q8_1 blocks (shapes validated by the caller).
-int run_mm_split(const void *w, const void *xq, float *y, int K, int N, int M, hipStream_t s) {
-    const bool gemv_ok = M <= kGemvMaxBatch && K <= kGemvMaxK && (int64_t)M * (K / kQK) * 48 <= 150 * 1024;
-    // The block_q4_0 AUTO dispatch's choices, each kernel reading the split layout: the
-    // GEMV up to batch 4 (one K slice) or 2, the LDS-resident skinny kernel for 5..16 at
-    // K <= 4096, the per-wave skinny kernel up to 16, then the K-sliced GEMM where it is
-    // faster than the tiled ones, the small-tile GEMM while the 128 x 128 tiles would not
-    // fill the chip well, else the 128 x 128 GEMM.
+int run_mm_split(const void *w, const void *xq, float *y, int K, int N, int M, int kernel, hipStream_t s) {
+    if (kernel == JJO_ALGO_AUTO) kernel = auto_kernel(w, xq, K, N, M, true);
+    if (kernel >= JJO_KERNEL_KSLICE) return run_kslice(w, xq, y, K, N, M, true, kernel - JJO_KERNEL_KSLICE, s);
     hipError_t e;
-    if (gemv_ok && M <= (K <= 4096 ? kGemvPreferredBatch : 2)) {
-        e = launch_gemv_q4s(w, xq, y, K, N, M, s);
-        return e == hipSuccess ? JJO_OK : hip_fail(e, "gemv_q4s launch");
+    switch (kernel) {
+        case JJO_ALGO_GEMV:
+            e = launch_gemv_q4s(w, xq, y, K, N, M, s);
+            return e == hipSuccess ? JJO_OK : hip_fail(e, "gemv_q4s launch");
+        case JJO_ALGO_SKINNY_LDS:
+            e = launch_gemm_skinny_persist_layout(w, xq, y, K, N, M, true, s);
+            return e == hipSuccess ? JJO_OK : hip_fail(e, "gemm_skinny_persist (split layout) launch");
+        case JJO_ALGO_SKINNY:
+            e = launch_gemm_skinny_layout(w, xq, y, K, N, M, true, s);
+            return e == hipSuccess ? JJO_OK : hip_fail(e, "gemm_skinny (split layout) launch");
+        case JJO_ALGO_MFMA64:
+        case JJO_ALGO_MFMA32:
+            e = launch_gemm_mfma64(w, xq, y, K, N, M, s, kernel == JJO_ALGO_MFMA32 ? 32 : 64, true);
+            return e == hipSuccess ? JJO_OK : hip_fail(e, "gemm_mfma64 (split layout) launch");
+        default:
+            e = launch_gemm_q4s_mfma(w, xq, y, K, N, M, true, s);
+            return e == hipSuccess ? JJO_OK : hip_fail(e, "gemm_q4s_mfma launch");
     }
-    if (K <= 4096 && M >= 5 && M <= 16 && gemm_skinny_persist_supported(w, xq, K, M)) {
-        e = launch_gemm_skinny_persist_layout(w, xq, y, K, N, M, true, s);
-        return e == hipSuccess ? JJO_OK : hip_fail(e, "gemm_skinny_persist (split layout) launch");
-    }
-    if (M <= 16 && gemm_skinny_supported(w, xq, K, M)) {
-        e = launch_gemm_skinny_layout(w, xq, y, K, N, M, true, s);
-        return e == hipSuccess ? JJO_OK : hip_fail(e, "gemm_skinny (split layout) launch");
-    }
-    if (gemv_ok) {
-        e = launch_gemv_q4s(w, xq, y, K, N, M, s);
-        return e == hipSuccess ? JJO_OK : hip_fail(e, "gemv_q4s launch");
-    }
-    if (const int shape = kslice_shape(K, N, M); shape >= 0) return run_kslice(w, xq, y, K, N, M, true, shape, s);
-    if (gemm_skinny_supported(w, xq, K, M)) {
-        e = launch_gemm_skinny_layout(w, xq, y, K, N, M, true, s);
-        return e == hipSuccess ? JJO_OK : hip_fail(e, "gemm_skinny (split layout) launch");
-    }
-    if (const int tr = small_tile_rows(N, M); tr != 0) {
-        e = launch_gemm_mfma64(w, xq, y, K, N, M, s, tr, true);
-        return e == hipSuccess ? JJO_OK : hip_fail(e, "gemm_mfma64 (split layout) launch");
-    }
-    e = launch_gemm_q4s_mfma(w, xq, y, K, N, M, true, s);
-    return e == hipSuccess ? JJO_OK : hip_fail(e, "gemm_q4s_mfma launch");
 }
 
 int validate_split(const void *w, const void *xq, const void *y, int K, int N, int M) {
@@ -504,7 +521,7 @@ int mat_mul_q4_0s_q8_1_device(const void *d_w_split, const void *d_x_q8_1, float
     int rc = validate_split(d_w_split, d_x_q8_1, d_y, ncols_k, nrows_out, batch);
     if (rc != JJO_OK) return rc;
     if ((rc = require_gfx950()) != JJO_OK) return rc;
-    return run_mm_split(d_w_split, d_x_q8_1, d_y, ncols_k, nrows_out, batch, (hipStream_t)stream);
+    return run_mm_split(d_w_split, d_x_q8_1, d_y, ncols_k, nrows_out, batch, JJO_ALGO_AUTO, (hipStream_t)stream);
 }
 
 int mat_mul_q4_0s_q8_1_f32_device(const void *d_w_split, const float *d_x, void *d_quant_workspace, float *d_y,
@@ -525,7 +542,7 @@ int mat_mul_q4_0s_q8_1_f32_device(const void *d_w_split, const float *d_x, void 
         return set_error(JJO_ERR_INVALID_ARG, "quant workspace is required when batch > 1");
     hipError_t e = launch_quantize_q8_1(d_x, d_quant_workspace, ncols_k, batch, 1, s);
     if (e != hipSuccess) return hip_fail(e, "quantize_q8_1 launch");
-    return run_mm_split(d_w_split, d_quant_workspace, d_y, ncols_k, nrows_out, batch, s);
+    return run_mm_split(d_w_split, d_quant_workspace, d_y, ncols_k, nrows_out, batch, JJO_ALGO_AUTO, s);
 }
 
 int mat_mul_q4_0_q8_1_block_sums_device(const void *d_w_q4_0, const void *d_x_q8_1, int32_t *d_sumi,
@@ -539,6 +556,32 @@ int mat_mul_q4_0_q8_1_block_sums_device(const void *d_w_q4_0, const void *d_x_q8
     hipError_t e = launch_block_sums(d_w_q4_0, d_x_q8_1, d_sumi, ncols_k, nrows_out, batch, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "block_sums launch");
     return JJO_OK;
+}
+
+int jjo_mm_auto_kernel(int ncols_k, int nrows_out, int batch, int split) {
+    clear_error();
+    const void *a = reinterpret_cast<const void *>(16);  // shapes and a 16-byte alignment decide
+    if (validate_mm(a, a, a, ncols_k, nrows_out, batch) != JJO_OK) return -1;
+    return auto_kernel(a, a, ncols_k, nrows_out, batch, split != 0);
+}
+
+int jjo_mm_kernel_device(const void *d_w, const void *d_x_q8_1, float *d_y, int ncols_k, int nrows_out, int batch,
+                         int split, int kernel, void *stream) {
+    clear_error();
+    int rc = split ? validate_split(d_w, d_x_q8_1, d_y, ncols_k, nrows_out, batch)
+                   : validate_mm(d_w, d_x_q8_1, d_y, ncols_k, nrows_out, batch);
+    if (rc != JJO_OK) return rc;
+    const bool sliced = kernel >= JJO_KERNEL_KSLICE;
+    const int shape = kernel - JJO_KERNEL_KSLICE;
+    if (sliced ? !kslice_accepts(shape, ncols_k, nrows_out, batch)
+               : kernel != JJO_ALGO_MFMA64 && kernel != JJO_ALGO_MFMA32 && kernel != JJO_ALGO_MFMA_W32)
+        return set_error(JJO_ERR_INVALID_ARG, "kernel %d does not run ncols_k=%d nrows_out=%d batch=%d", kernel, ncols_k,
+                         nrows_out, batch);
+    if ((rc = require_gfx950()) != JJO_OK) return rc;
+    hipStream_t s = (hipStream_t)stream;
+    if (sliced) return run_kslice(d_w, d_x_q8_1, d_y, ncols_k, nrows_out, batch, split != 0, shape, s);
+    return split ? run_mm_split(d_w, d_x_q8_1, d_y, ncols_k, nrows_out, batch, kernel, s)
+                 : run_mm(d_w, d_x_q8_1, d_y, ncols_k, nrows_out, batch, kernel, s);
 }
 
 int jjo_read_floor_device(const void *d_src, int64_t bytes, uint32_t *d_out, void *stream) {

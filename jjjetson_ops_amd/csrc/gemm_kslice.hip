@@ -444,19 +444,21 @@ hipError_t launch(const void *w, const void *xq, float *y, int K, int N, int M, 
     return hipGetLastError();
 }
 
-// The tile shapes with their estimated time: a launch runs in rounds of `resident`
-// workgroups per CU; a round costs round_us + stage_us per 128-value stage, a (last) round
-// of at most one workgroup per CU alone_us per stage.  Fitted to K=1024..14336, N=1024..14336,
-// 17..1024 tokens, both layouts; within about 10% of the measurements.
+// The tile shapes with their estimated time: a launch runs in rounds of `resident` workgroups
+// per CU; a round costs round_us + stage_us per 128-value stage, a (last) round of at most one
+// workgroup per CU alone_us + alone_stage_us per stage, of which `idle` is left when the chip is
+// nearly empty.  Fitted to K=128..14336, N=256..151936, 17..3072 tokens, the mean of the two
+// layouts (they differ by 2-6%, and one table gives both the same shape and so the same bits):
+// an estimate is off by 7-10% (one standard deviation), 15-20% for one in twenty.
 struct Shape {
     int rt, ct, resident;
-    double fixed_us, round_us, stage_us, alone_us;
+    double fixed, round_us, stage_us, alone_us, alone_stage_us, idle;
 };
 constexpr Shape kShapes[] = {
-    {1, 1, 2, 3.5, 0.5, 0.300, 0.185},  // 8 waves (N=4096, K=4096, 64 tokens: 8.4 us)
-    {1, 2, 1, 2.0, 3.2, 0.210, 0.210},  // 8 waves (100 tokens: 11.9)
-    {2, 2, 1, 2.0, 3.0, 0.420, 0.420},  // 8 waves (256 tokens: 18.5)
-    {2, 2, 2, 3.0, 3.2, 0.775, 0.530},  // 4 waves (512 tokens: 30.7)
+    {1, 1, 2, 2.45, 1.26, 0.238, 0.777, 0.151, 0.812},  // 8 waves (N=4096, K=4096, 48 tokens: 8.6 / 8.2 us)
+    {1, 2, 1, 1.83, 2.14, 0.225, 2.14, 0.225, 1.0},     // 8 waves (100 tokens: 11.7 / 11.3)
+    {2, 2, 1, 2.55, 2.67, 0.362, 2.67, 0.365, 1.0},     // 8 waves (N=8192, 128 tokens: 17.8 / 17.2)
+    {2, 2, 2, 2.31, 2.76, 0.682, 2.76, 0.394, 1.0},     // 4 waves (512 tokens: 27.7 / 27.1)
 };
 
 }  // namespace
@@ -469,8 +471,9 @@ int kslice_pick(int K, int N, int M, double *us) {
         const int64_t g = (((int64_t)N + 32 * s.rt - 1) / (32 * s.rt)) * (((int64_t)M + 32 * s.ct - 1) / (32 * s.ct));
         const int64_t slots = s.resident * cus, rem = g % slots;
         const double stages = K / kQSuper, round = s.round_us + s.stage_us * stages;
-        const double t = s.fixed_us + (double)(g / slots) * round +
-                         (rem == 0 ? 0.0 : rem > cus ? round : s.round_us + s.alone_us * stages);
+        const double busy = g < cus ? (double)g / cus : 1.0;
+        const double alone = s.alone_us + s.alone_stage_us * stages * (s.idle + (1.0 - s.idle) * busy);
+        const double t = s.fixed + (double)(g / slots) * round + (rem == 0 ? 0.0 : rem > cus ? round : alone);
         if (i == 0 || t < *us) {
             best = i;
             *us = t;
