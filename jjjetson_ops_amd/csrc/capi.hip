@@ -204,11 +204,6 @@ double tiled_us(int K, int N, int M, bool split) {
            (double)((2 * halved + slots - 1) / slots) * (round + (split ? 1.60 : 1.47) * stages);
 }
 
-// A K-sliced tile shape runs a problem: 32-bit offsets inside a tile, tokens of one superblock.
-bool kslice_accepts(int shape, int K, int N, int M) {
-    return shape >= 0 && shape <= 3 && M <= 65535 && K < kMaxTileK;
-}
-
 // The K-sliced mid-batch kernel's tile shape where it is estimated to beat the tiled GEMMs,
 // else -1.  Measured, tiled against the best K-sliced shape (block_q4_0 / split, us): N=4096,
 // K=4096: 48 tokens 21.9 / 21.2 against 8.6 / 8.2, 512: 33.5 / 32.7 against 27.7 / 27.1, 1536: 85.2

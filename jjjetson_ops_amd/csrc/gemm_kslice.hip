@@ -437,8 +437,7 @@ hipError_t launch(const void *w, const void *xq, float *y, int K, int N, int M, 
     hipError_t e = ensure_dynamic_lds((const void *)kern, lds);
     if (e != hipSuccess) return e;
     const int64_t rows = ((int64_t)N + 32 * RT - 1) / (32 * RT), toks = ((int64_t)M + 32 * CT - 1) / (32 * CT);
-    const int64_t grid = (rows * toks + 7) / 8 * 8;
-    if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
+    const int64_t grid = (rows * toks + 7) / 8 * 8;  // kslice_accepts bounds it
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * WK), lds, stream, (const uint8_t *)w,
                        (const uint8_t *)xq, y, K, N, M, (int)rows, (int)toks);
     return hipGetLastError();
@@ -451,25 +450,36 @@ hipError_t launch(const void *w, const void *xq, float *y, int K, int N, int M, 
 // layouts (they differ by 2-6%, and one table gives both the same shape and so the same bits):
 // an estimate is off by 7-10% (one standard deviation), 15-20% for one in twenty.
 struct Shape {
-    int rt, ct, resident;
+    int rt, ct, waves, resident;
     double fixed, round_us, stage_us, alone_us, alone_stage_us, idle;
 };
 constexpr Shape kShapes[] = {
-    {1, 1, 2, 2.45, 1.26, 0.238, 0.777, 0.151, 0.812},  // 8 waves (N=4096, K=4096, 48 tokens: 8.6 / 8.2 us)
-    {1, 2, 1, 1.83, 2.14, 0.225, 2.14, 0.225, 1.0},     // 8 waves (100 tokens: 11.7 / 11.3)
-    {2, 2, 1, 2.55, 2.67, 0.362, 2.67, 0.365, 1.0},     // 8 waves (N=8192, 128 tokens: 17.8 / 17.2)
-    {2, 2, 2, 2.31, 2.76, 0.682, 2.76, 0.394, 1.0},     // 4 waves (512 tokens: 27.7 / 27.1)
+    {1, 1, 8, 2, 2.45, 1.26, 0.238, 0.777, 0.151, 0.812},  // N=4096, K=4096, 48 tokens: 8.6 / 8.2 us
+    {1, 2, 8, 1, 1.83, 2.14, 0.225, 2.14, 0.225, 1.0},     // 100 tokens: 11.7 / 11.3
+    {2, 2, 8, 1, 2.55, 2.67, 0.362, 2.67, 0.365, 1.0},     // N=8192, 128 tokens: 17.8 / 17.2
+    {2, 2, 4, 2, 2.31, 2.76, 0.682, 2.76, 0.394, 1.0},     // N=4096, 512 tokens: 27.7 / 27.1
 };
 
+int64_t shape_tiles(const Shape &s, int N, int M) {
+    return (((int64_t)N + 32 * s.rt - 1) / (32 * s.rt)) * (((int64_t)M + 32 * s.ct - 1) / (32 * s.ct));
+}
+
 }  // namespace
+
+// A launch holds less than 2^32 threads in x: 2^23 workgroups of eight waves, which one tile
+// per 32 rows and tokens reaches at N = 2^28, 17 tokens.
+bool kslice_accepts(int shape, int K, int N, int M) {
+    if (shape < 0 || shape >= (int)(sizeof(kShapes) / sizeof(kShapes[0])) || M > 65535 || K >= kMaxTileK) return false;
+    const Shape &s = kShapes[shape];
+    return (shape_tiles(s, N, M) + 7) / 8 * 8 * 64 * s.waves < 1LL << 32;
+}
 
 int kslice_pick(int K, int N, int M, double *us) {
     const int64_t cus = device_cu_count();
     int best = 0;
     for (int i = 0; i < (int)(sizeof(kShapes) / sizeof(kShapes[0])); ++i) {
         const Shape &s = kShapes[i];
-        const int64_t g = (((int64_t)N + 32 * s.rt - 1) / (32 * s.rt)) * (((int64_t)M + 32 * s.ct - 1) / (32 * s.ct));
-        const int64_t slots = s.resident * cus, rem = g % slots;
+        const int64_t g = shape_tiles(s, N, M), slots = s.resident * cus, rem = g % slots;
         const double stages = K / kQSuper, round = s.round_us + s.stage_us * stages;
         const double busy = g < cus ? (double)g / cus : 1.0;
         const double alone = s.alone_us + s.alone_stage_us * stages * (s.idle + (1.0 - s.idle) * busy);
@@ -484,6 +494,7 @@ int kslice_pick(int K, int N, int M, double *us) {
 
 hipError_t launch_gemm_kslice(const void *w, const void *xq, float *y, int K, int N, int M, bool split, int shape,
                               hipStream_t stream) {
+    if (!kslice_accepts(shape, K, N, M)) return hipErrorInvalidValue;
     switch (shape) {
         case 0: return launch<1, 1, 8, 4>(w, xq, y, K, N, M, split, stream);
         case 1: return launch<1, 2, 8, 2>(w, xq, y, K, N, M, split, stream);

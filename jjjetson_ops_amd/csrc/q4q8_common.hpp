@@ -96,8 +96,9 @@ hipError_t launch_gemm_mfma64(const void *w, const void *xq, float *y, int K, in
                               hipStream_t stream, int tile_rows, bool split = false);
 // Mid-batch GEMM, K cut over the waves of a workgroup (either layout; block_q4_0 4-byte,
 // split 16-byte aligned weights, any K % 128 == 0).  kslice_pick returns the tile shape
-// for a problem and its estimated time in microseconds.
+// for a problem and its estimated time in microseconds, kslice_accepts whether a shape can run it.
 int kslice_pick(int K, int N, int M, double *us);
+bool kslice_accepts(int shape, int K, int N, int M);
 hipError_t launch_gemm_kslice(const void *w, const void *xq, float *y, int K, int N, int M, bool split, int shape,
                               hipStream_t stream);
 // Its grouped form (experts' row tiles x tiles of 32 * cols routes, cols 1 or 2).  midq == nullptr: the

@@ -36,6 +36,22 @@ def test_kslice(K, N, M, form):
         assert capi.mm_auto_kernel(K, N, M, split) == capi.KERNEL_KSLICE + form
 
 
+@pytest.mark.parametrize("K,N,M", [(1536, 1 << 28, 17), (1536, 1 << 28, 32), (2048, 1 << 27, 64), (256, 1 << 28, 20)])
+def test_launch_fits_the_grid(K, N, M):
+    """A launch holds less than 2^32 threads in x; a K-sliced tile is a workgroup of 512
+    threads (forms 0..2) or 256, in multiples of eight workgroups."""
+    tile = ((32, 32, 512), (32, 64, 512), (64, 64, 512), (64, 64, 256))
+    for split in BOTH:
+        form = capi.mm_auto_kernel(K, N, M, split) - capi.KERNEL_KSLICE
+        if form >= 0:
+            rows, toks, threads = tile[form]
+            assert (-(-N // rows) * -(-M // toks) + 7) // 8 * 8 * threads < 1 << 32
+    a16 = ctypes.c_void_p(16)  # refused before any device is touched
+    assert capi.lib().jjo_mm_kernel_device(a16, a16, a16, 1536, 1 << 28, 17, 0, capi.KERNEL_KSLICE,
+                                           None) == capi.JJO_ERR_INVALID_ARG
+    assert capi.mm_auto_kernel(1536, (1 << 28) - 256, 17) == capi.KERNEL_KSLICE  # the most that fits
+
+
 def test_invalid_calls_are_refused():
     with pytest.raises(capi.JJOError):
         capi.mm_auto_kernel(96, 4, 1)
