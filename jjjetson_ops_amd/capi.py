@@ -271,7 +271,12 @@ def _linear(split: bool, x, w, y, in_features, out_features, num_tokens, ws, str
         lib()  # the same loud failure where nothing is built
         from ._linear import linear
         _linear_native = linear
-    return _linear_native(split, _current_stream, x, w, y, in_features, out_features, num_tokens, ws, stream)
+    rc = _linear_native(split, _current_stream, x, w, y, in_features, out_features, num_tokens, ws, stream)
+    if rc is None:  # an argument that only ctypes converts (a c_int, _as_parameter_) or refuses (ArgumentError)
+        fn = lib().linear_q4_0s_forward_device if split else lib().linear_q4_0_forward_device
+        rc = fn(_stream(stream), None if ws is None else _dev(ws, "ws"), _dev(x, "x"), _dev(w, "w"), _dev(y, "y"),
+                in_features, out_features, num_tokens)
+    return rc
 
 
 def quantize_q8_1(x, out, dims=None, stream=None) -> None:

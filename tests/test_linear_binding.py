@@ -5,6 +5,8 @@ if __name__ == "__main__":  # `python tests/<file>.py`, as the reference runs it
 
     import pytest as _pytest
     _sys.exit(_pytest.main([__file__, "-q"]))
+import ctypes
+
 import numpy as np
 import pytest
 import torch  # before the library: both then share torch's HIP runtime
@@ -34,12 +36,29 @@ def test_linear_binding_errors(entry):
                 entry(*args, 128, 4, 1, stream=0)
         with pytest.raises(ValueError, match="ws " + text):
             entry(ok, ok, ok, 128, 4, 1, ws=bad, stream=0)
-    with pytest.raises(TypeError):
-        entry(ok, ok, ok, 128.0, 4, 1, stream=0)
+    for k in range(3):
+        args = [128, 4, 1]
+        args[k] = float(args[k])
+        with pytest.raises(ctypes.ArgumentError, match=f"argument {6 + k}"):  # as from every other entry
+            entry(ok, ok, ok, *args, stream=0)
     with pytest.raises(AttributeError):
         entry(None, ok, ok, 128, 4, 1, stream=0)
     with pytest.raises(capi.JJOError) as e:  # refused before any device is touched
         entry(ok, ok, ok, 128, 0, 1, stream=0)
+    assert e.value.code == capi.JJO_ERR_INVALID_ARG and "out_features=0" in str(e.value)
+
+
+class AsParameter:
+    _as_parameter_ = ctypes.c_int(0)
+
+
+@pytest.mark.parametrize("entry", [capi.linear_q4_0, capi.linear_q4_0_split])
+@pytest.mark.parametrize("zero", [np.int64(0), False, 1 << 32, ctypes.c_int(0), AsParameter()])
+def test_linear_binding_ints(entry, zero):
+    """A size may be whatever ctypes takes for a C int; the entry refuses the zero itself."""
+    ok = Fake()
+    with pytest.raises(capi.JJOError) as e:
+        entry(ok, ok, ok, 128, zero, 1, stream=0)
     assert e.value.code == capi.JJO_ERR_INVALID_ARG and "out_features=0" in str(e.value)
 
 
