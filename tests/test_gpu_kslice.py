@@ -1,8 +1,8 @@
-"""The K-sliced mid-batch GEMM through the AUTO entries, both weight layouts, against
-the CPU oracle: each of its tile shapes (chosen by the output's size), row and token
-tails, fewer 128-value stages than waves, uneven slices and 4-byte-aligned weights.
-The layouts share every instruction after the operand expansion, so their results are
-equal bit for bit."""
+"""The K-sliced mid-batch GEMM, both weight layouts, against the CPU oracle: each of its
+tile forms at row and token tails, fewer 128-value stages than waves and uneven slices,
+asked for by name; the form the entries choose, with 4-byte-aligned weights; the grouped
+form.  The layouts share every instruction after the operand expansion, so their results
+are equal bit for bit."""
 if __name__ == "__main__":  # `python tests/<file>.py`, as the reference runs its tests
     import sys as _sys
 
@@ -18,37 +18,62 @@ pytestmark = pytest.mark.gpu
 RTOL, ATOL = 1e-3, 1e-4  # the repository's bar against the oracle's fp64 sums
 
 
-@pytest.mark.parametrize("K,N,M", [
-    # 32 x 32 tiles, 8 waves: one stage for 8 waves; 3, 9 and 32 stages; tails
-    (128, 1, 17), (128, 33, 31), (384, 95, 33), (1152, 160, 64), (4096, 64, 65), (1152, 257, 32),
-    # 32 x 64, 8 waves
-    (256, 2077, 129), (1280, 2080, 160),
-    # 64 x 64, 8 waves
-    (256, 2075, 389), (1152, 2080, 400),
-    # 64 x 64, 4 waves
-    (256, 4070, 500), (640, 4096, 512),
-])
-def test_kslice_shapes(K, N, M, dev):
+def _case(K, N, M, dev):
+    """(expected, block_q4_0 weights, the same in the split layout, activation blocks)"""
     import torch
-    print(f"[case] kslice K={K} N={N} M={M}", flush=True)
     rng = np.random.default_rng(K + N * M)
     w = c_oracle.quantize_q4_0((rng.standard_normal((N, K)) * 0.02).astype(np.float32))
     xq = c_oracle.quantize_q8_1(rng.standard_normal((M, K)).astype(np.float32), [K, M])
-    exp = c_oracle.matmul(w, xq, K, N, M)
-    xq_d = torch.from_numpy(xq).to(dev)
-    w_pad = torch.zeros(w.size + 16, dtype=torch.uint8, device=dev)
-    w_pad[4:4 + w.size] = torch.from_numpy(w).to(dev)
+    w_d = torch.from_numpy(w).to(dev)
     ws = torch.empty(w.size, dtype=torch.uint8, device=dev)
-    capi.q4_0_to_split(torch.from_numpy(w).to(dev), ws, N, K)
-    got = []
-    for run, wt in ((capi.mat_mul, torch.from_numpy(w).to(dev)), (capi.mat_mul, w_pad[4:4 + w.size]),
-                    (capi.mat_mul_split, ws)):
-        y = torch.full((M * N + 64,), float("nan"), dtype=torch.float32, device=dev)
-        run(wt, xq_d, y, K, N, M)
-        torch.cuda.synchronize()
-        assert torch.isnan(y[M * N:]).all()  # nothing past the output
-        got.append(y[:M * N].cpu().numpy().reshape(M, N))
-        np.testing.assert_allclose(got[-1], exp, rtol=RTOL, atol=ATOL)
+    capi.q4_0_to_split(w_d, ws, N, K)
+    return c_oracle.matmul(w, xq, K, N, M), w_d, ws, torch.from_numpy(xq).to(dev)
+
+
+def _run(fn, M, N, dev):
+    """fn(y); the result, after a look at what lies past it."""
+    import torch
+    y = torch.full((M * N + 64,), float("nan"), dtype=torch.float32, device=dev)
+    fn(y)
+    torch.cuda.synchronize()
+    assert torch.isnan(y[M * N:]).all()
+    return y[:M * N].cpu().numpy().reshape(M, N)
+
+
+@pytest.mark.parametrize("form", [0, 1, 2, 3])
+@pytest.mark.parametrize("K,N,M", [
+    (128, 1, 1), (128, 33, 65),      # one stage for four or eight waves; one row or token in a tile
+    (384, 95, 31), (640, 130, 97),   # 3 and 5 stages; tails of 31 and 2 rows, 31 and 33 tokens
+    (1152, 161, 64), (1280, 64, 33), # 9 and 10 stages; N % 4 == 1; full tiles
+    (2176, 127, 130), (4096, 66, 32),
+])
+def test_kslice_forms(K, N, M, form, dev):
+    """Forms 0..3: 32 x 32, 32 x 64 and 64 x 64 tiles of eight waves, 64 x 64 of four."""
+    print(f"[case] kslice form={form} K={K} N={N} M={M}", flush=True)
+    exp, w, ws, xq = _case(K, N, M, dev)
+    kernel = capi.KERNEL_KSLICE + form
+    got = [_run(lambda y: capi.mm_kernel(wt, xq, y, K, N, M, kernel, split), M, N, dev)
+           for wt, split in ((w, False), (ws, True))]
+    np.testing.assert_allclose(got[0], exp, rtol=RTOL, atol=ATOL)
+    assert np.array_equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("K,N,M,form", [
+    (128, 33, 31, 0), (384, 95, 33, 0), (4096, 64, 65, 0), (2944, 4106, 33, 1), (768, 6325, 97, 2),
+    (640, 3591, 199, 3), (640, 8095, 98, 3),
+])
+def test_kslice_chosen(K, N, M, form, dev):
+    """Shapes that the entries give to each form, with weights at the least alignment."""
+    import torch
+    print(f"[case] kslice K={K} N={N} M={M}", flush=True)
+    for split in (False, True):
+        assert capi.mm_auto_kernel(K, N, M, split) == capi.KERNEL_KSLICE + form
+    exp, w, ws, xq = _case(K, N, M, dev)
+    w_pad = torch.zeros(w.numel() + 16, dtype=torch.uint8, device=dev)
+    w_pad[4:4 + w.numel()] = w
+    got = [_run(lambda y: run(wt, xq, y, K, N, M), M, N, dev)
+           for run, wt in ((capi.mat_mul, w), (capi.mat_mul, w_pad[4:4 + w.numel()]), (capi.mat_mul_split, ws))]
+    np.testing.assert_allclose(got[0], exp, rtol=RTOL, atol=ATOL)
     assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
 
 

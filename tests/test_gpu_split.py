@@ -132,10 +132,12 @@ def test_split_f32_batch(M, dev):
                                    # K % 256 != 0: the skinny kernel is unsupported, batch 3/6 take
                                    # the GEMV (two K slices), batch 12 the GEMM
                                    (4224, 100, 3), (4224, 100, 6), (4224, 100, 12),
-                                   # the per-wave skinny kernel (batch 17..32; 3..16 above K = 4096)
-                                   (4096, 300, 24), (4096, 1000, 32), (11008, 257, 3), (14336, 200, 9),
-                                   # the small-tile GEMM, 32- and 64-row tiles
-                                   (4096, 4096, 48), (4096, 1000, 64), (14336, 520, 200)])
+                                   # the per-wave skinny kernel (batch 3..16 above K = 4096; 17..32
+                                   # on short rows with many outputs)
+                                   (11008, 257, 3), (14336, 200, 9), (256, 40003, 32), (256, 65537, 17),
+                                   # the K-sliced GEMM
+                                   (4096, 300, 24), (4096, 1000, 32), (4096, 4096, 48), (4096, 1000, 64),
+                                   (14336, 520, 200)])
 def test_split_gemm(K, N, M, dev):
     import torch
     note(f"split gemm M={M} K={K} N={N}")
@@ -149,21 +151,51 @@ def test_split_gemm(K, N, M, dev):
     np.testing.assert_allclose(host(y).reshape(M, N), c_oracle.matmul(w, xq, K, N, M), rtol=RTOL, atol=ATOL)
 
 
-@pytest.mark.parametrize("K,N,M", [(256, 5120, 1700), (256, 14336, 2048), (128, 128 * 33, 128 * 16 + 5)])
-def test_split_gemm_tail_round(K, N, M, dev):
+@pytest.mark.parametrize("kernel", [capi.ALGO_MFMA32, capi.ALGO_MFMA64, capi.ALGO_MFMA_W32])
+@pytest.mark.parametrize("K,N,M", [(128, 1, 1), (128, 129, 65), (384, 127, 33), (640, 161, 130), (1152, 64, 257),
+                                   (4096, 300, 96)])
+def test_split_tiles(K, N, M, kernel, dev):
+    """The tiled GEMMs by name (32- and 64-row tiles, 128 x 128) on a split layout, at row
+    and token tails, one stage and odd stage counts; few 128 x 128 tiles run as half tiles."""
+    import torch
+    note(f"split tiles kernel={kernel} M={M} K={K} N={N}")
+    rng = np.random.default_rng(K + 3 * N + M)
+    w = _weights(rng, N, K)
+    xq = c_oracle.quantize_q8_1(rng.standard_normal((M, K)).astype(np.float32), [K, M])
+    y = torch.full((M * N + 64,), float("nan"), dtype=torch.float32, device=dev)
+    capi.mm_kernel(split_dev(w, N, K, dev), to_dev(xq, dev), y, K, N, M, kernel, split=True)
+    got = host(y)
+    assert np.isnan(got[M * N:]).all()
+    np.testing.assert_allclose(got[:M * N].reshape(M, N), c_oracle.matmul(w, xq, K, N, M), rtol=RTOL, atol=ATOL)
+
+
+@pytest.mark.parametrize("K,N,M,kernel", [(256, 5120, 1700, 0), (256, 14336, 2048, 0),
+                                          (128, 128 * 33, 128 * 16 + 5, 0),
+                                          # the 128 x 128 kernel by name: 561 tiles, 49 as halves, half of
+                                          # those without a token; 800 whole ones, 1, 33, 68 or 97 tokens in the last
+                                          (128, 128 * 33, 128 * 16 + 5, capi.ALGO_MFMA_W32),
+                                          (128, 12800, 897, capi.ALGO_MFMA_W32),
+                                          (384, 12797, 896 + 33, capi.ALGO_MFMA_W32),
+                                          (128, 12797, 896 + 68, capi.ALGO_MFMA_W32),
+                                          (256, 12800, 896 + 97, capi.ALGO_MFMA_W32)])
+def test_split_gemm_tail_round(K, N, M, kernel, dev):
     """Tile counts that leave a partial last round of at most half the 512 slots
     (2 per CU): that round runs as 64-token half tiles, including a half that lies
-    entirely past M.  Checked on a row subset that includes both ends of every
-    128-row tile boundary touched."""
+    entirely past M; and a full round with a token tail in its tiles.  Checked on a row
+    subset that includes both ends of every 128-row tile boundary touched.  kernel 0:
+    what the entry chooses (64 x 64 tiles; the 128 x 128 kernel; 64 x 64)."""
     import torch
-    note(f"split gemm tail round M={M} K={K} N={N}")
+    note(f"split gemm tail round M={M} K={K} N={N} kernel={kernel}")
     rng = np.random.default_rng(K + N + M)
     w = _weights(rng, N, K)
     x = rng.standard_normal((M, K)).astype(np.float32)
     xq = c_oracle.quantize_q8_1(x, [K, M])
     ws = split_dev(w, N, K, dev)
     y = torch.full((M * N,), float("nan"), dtype=torch.float32, device=dev)
-    capi.mat_mul_split(ws, to_dev(xq, dev), y, K, N, M)
+    if kernel:
+        capi.mm_kernel(ws, to_dev(xq, dev), y, K, N, M, kernel, split=True)
+    else:
+        capi.mat_mul_split(ws, to_dev(xq, dev), y, K, N, M)
     got = host(y).reshape(M, N)
     rows = np.unique(np.concatenate([rng.choice(N, 200, replace=False), [0, 127, 128, N - 129, N - 128, N - 1]]))
     nb = K // 32
