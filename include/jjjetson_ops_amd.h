@@ -198,6 +198,13 @@ int mat_mul_q4_0_q8_1_block_sums_device(const void *d_w_q4_0, const void *d_x_q8
 int jjo_mm_auto_kernel(int ncols_k, int nrows_out, int batch, int split);
 int jjo_mm_kernel_device(const void *d_w, const void *d_x_q8_1, float *d_y, int ncols_k, int nrows_out,
                          int batch, int split, int kernel, void *stream);
+/* The same for the grouped entries (nrows_out: 2 * intermediate_size for gate|up): JJO_ALGO_GEMV
+ * (routed), JJO_ALGO_MFMA (tiles of 128 routes) or JJO_KERNEL_KSLICE + 1 or 2 (32-route
+ * column tiles of a workgroup); -1 for an invalid shape.  The last two can be chosen. */
+int jjo_grouped_auto_kernel(int ncols_k, int nrows_out, int n_routes, int n_experts);
+int jjo_grouped_kernel_device(const void *d_w, const void *d_x_q8_1, const int32_t *d_expert_offsets, int n_experts,
+                              const int32_t *d_route_dst, float *d_y, int ncols_k, int nrows_out, int n_routes,
+                              int split, int kernel, void *stream);
 
 /*
  * DIAGNOSTIC ONLY (a measurement probe, not part of the drop-in path; no

@@ -26,7 +26,7 @@ ALGO_SKINNY_LDS = 4
 ALGO_MFMA64 = 5
 ALGO_MFMA32 = 6
 ALGO_MFMA_W32 = 7
-KERNEL_KSLICE = 16  # + tile form 0..3 (mm_auto_kernel, mm_kernel)
+KERNEL_KSLICE = 16  # + tile form 0..3 (mm_auto_kernel, mm_kernel), column tiles (grouped_auto_kernel)
 
 QK = 32
 QSUPER = 128
@@ -49,6 +49,8 @@ EXPORTED_SYMBOLS = (
     "mat_mul_q4_0_q8_1_grouped_device",
     "mat_mul_q4_0s_q8_1_grouped_device",
     "jjo_mm_auto_kernel",
+    "jjo_grouped_auto_kernel",
+    "jjo_grouped_kernel_device",
     "jjo_mm_kernel_device",
     "jjo_read_floor_device",
     "linear_q4_0_workspace_bytes",
@@ -146,6 +148,10 @@ def lib() -> ctypes.CDLL:
         L.mat_mul_q4_0s_q8_1_grouped_device.argtypes = [vp, vp, vp, i32, vp, vp, i32, i32, i32, vp]
         L.jjo_mm_auto_kernel.restype = i32
         L.jjo_mm_auto_kernel.argtypes = [i32, i32, i32, i32]
+        L.jjo_grouped_auto_kernel.restype = i32
+        L.jjo_grouped_auto_kernel.argtypes = [i32, i32, i32, i32]
+        L.jjo_grouped_kernel_device.restype = i32
+        L.jjo_grouped_kernel_device.argtypes = [vp, vp, vp, i32, vp, vp, i32, i32, i32, i32, i32, vp]
         L.jjo_mm_kernel_device.restype = i32
         L.jjo_mm_kernel_device.argtypes = [vp, vp, vp, i32, i32, i32, i32, i32, vp]
         L.jjo_read_floor_device.restype = i32
@@ -399,6 +405,17 @@ def grouped_mat_mul(w, xq, expert_offsets, y, K: int, N: int, n_routes: int, rou
                     stream=None, split: bool = False) -> None:
     """One-launch MoE expert GEMM over routes sorted by expert (see the C header);
     split: w holds the stacked experts repacked into the split layout."""
+    _grouped(w, xq, expert_offsets, y, K, N, n_routes, route_dst, stream, split, 0)
+
+
+def grouped_kernel(w, xq, expert_offsets, y, K: int, N: int, n_routes: int, kernel: int, route_dst=None,
+                   stream=None, split: bool = False) -> None:
+    """jjo_grouped_kernel_device: grouped_mat_mul on one of the kernels that grouped_auto_kernel
+    names (but ALGO_GEMV)."""
+    _grouped(w, xq, expert_offsets, y, K, N, n_routes, route_dst, stream, split, kernel)
+
+
+def _grouped(w, xq, expert_offsets, y, K, N, n_routes, route_dst, stream, split, kernel) -> None:
     import torch
     n_experts = expert_offsets.numel() - 1
     if expert_offsets.dtype != torch.int32:
@@ -408,6 +425,11 @@ def grouped_mat_mul(w, xq, expert_offsets, y, K: int, N: int, n_routes: int, rou
     if w.numel() * w.element_size() < n_experts * N * (K // QK) * Q4_BLOCK_BYTES:
         raise ValueError("weight buffer too small for all experts")
     rd = _dev(route_dst, "route_dst") if route_dst is not None else ctypes.c_void_p(0)
+    if kernel:
+        _check(lib().jjo_grouped_kernel_device(_dev(w, "w"), _dev(xq, "xq"), _dev(expert_offsets, "offsets"), n_experts,
+                                               rd, _dev(y, "y"), K, N, n_routes, int(split), kernel, _stream(stream)),
+               "jjo_grouped_kernel_device")
+        return
     fn = lib().mat_mul_q4_0s_q8_1_grouped_device if split else lib().mat_mul_q4_0_q8_1_grouped_device
     _check(fn(_dev(w, "w"), _dev(xq, "xq"), _dev(expert_offsets, "offsets"), n_experts, rd, _dev(y, "y"), K, N,
               n_routes, _stream(stream)), "grouped_mat_mul")
@@ -419,6 +441,14 @@ def mm_auto_kernel(K: int, N: int, M: int, split: bool = False) -> int:
     k = int(lib().jjo_mm_auto_kernel(K, N, M, int(split)))
     if k < 0:
         _check(JJO_ERR_INVALID_ARG, "jjo_mm_auto_kernel")
+    return k
+
+
+def grouped_auto_kernel(K: int, N: int, n_routes: int, n_experts: int) -> int:
+    """jjo_grouped_auto_kernel: ALGO_GEMV, ALGO_MFMA or KERNEL_KSLICE + column tiles."""
+    k = int(lib().jjo_grouped_auto_kernel(K, N, n_routes, n_experts))
+    if k < 0:
+        _check(JJO_ERR_INVALID_ARG, "jjo_grouped_auto_kernel")
     return k
 
 

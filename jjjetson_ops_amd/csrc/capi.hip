@@ -9,6 +9,8 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
+#include <cmath>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -610,23 +612,54 @@ int mean_routes(int n_routes, int n_experts) {
 }
 // 32-route column tiles of the K-sliced grouped GEMM (one or two per workgroup), or 0 for
 // the 128-route tiles.  A 128-route tile with a handful of routes stages 128 weight rows for
-// one 32-column strip and is bound by that latency; the K-sliced form reads an expert's
-// weights with four waves per 64 rows.  FFN, us, 128-route tiles -> one / two column tiles
-// (block_q4_0): E=64 top-8 H=2048 I=1408, mean 2: 138 -> 124 / 132, 12.5: 158 -> 137 / 144,
-// 32: 210 -> 189 / 188, 64: 283 -> 293 / 279; E=8 top-2 H=4096 I=14336, mean 8: 292 -> 229
-// / 243, 25: 323 -> 248 / 262, 32: 475 -> 375 / 313, 64: 554 -> 542 / 488, 128: 798 -> 928 /
-// 804.  The mean hides the skew of a random router: from about 24 on, most launches hold
-// an expert above 32 routes, whose weights one column tile reads twice.
-int grouped_kslice_cols(int n_routes, int n_experts, int K) {
-    if (K >= kMaxTileK) return 0;
-    const int mean = mean_routes(n_routes, n_experts);
-    return mean <= 24 ? 1 : mean <= 80 ? 2 : 0;
+// one 32-column strip and, with few of them in flight, is bound by that latency; the K-sliced
+// form reads an expert's weights with four waves per 64 rows.  On short rows its waves
+// have a stage or none each, and where the 128-route tiles fill the chip it reads the
+// weights and the activation more often.  Measured (us, 128-route tiles against one / two
+// column tiles, block_q4_0): 8 experts, K=4096, N=1024, mean 48: 61 against 16.5 / 20.7; 64
+// experts, K=2048, N=2816, mean 32: 93 against 91 / 82, mean 80: 143 against 171 / 156; K=1024,
+// N=4096, mean 48: 90 against 99 / 82; K=256, N=4096, mean 16: 28 against 34 / 34; K=128,
+// N=14336, mean 7: 71 against 100 / 99, mean 80: 132 against 307 / 247.
+//   A kernel's time is estimated as fixed + hypot(latency, work): the stages of one tile,
+// and the launch's row tiles x token tiles (and 32-route columns) per CU.  An expert's routes are
+// not known here: the token tiles are those expected of a normal spread about the mean, a
+// Poisson one's and 15% of the mean.  Fitted to 9000 launches on weights that no cache holds
+// (K=128..14336, N=64..28672, 2 to 256 experts, means 2 to 100, balanced and skewed routers, both
+// layouts, with and without SwiGLU), off by 9-11% (one standard deviation), 13-18% with
+// a skewed router; the K-sliced form has to be estimated 3% lower.  On 13000 others, of means up
+// to 80, the choice is 1.5% from the best kernel on average, takes 0.69 of the 128-route tiles'
+// time and is slower than those by more than 3% for 2.7% of the launches, by more than 10% for
+// 0.8%; with lines at means of 24 and 80 alone: 0.72, 13.7% and 8.8%.
+//   Both layouts take the same kernel, so their results are the same bits.
+int grouped_kslice_cols(int n_routes, int n_experts, int K, int N) {
+    if (K >= kMaxTileK || mean_routes(n_routes, n_experts) > 80) return 0;
+    const double active = n_experts < n_routes ? n_experts : n_routes, mean = n_routes / active;
+    const double spread = std::sqrt(2.0 * (mean + 0.0225 * mean * mean));
+    auto above = [&](int routes) { return 0.5 * std::erfc((routes + 0.5 - mean) / spread); };
+    auto tiles = [&](int routes) {  // of all experts: expected ceil(expert's routes / routes)
+        double n = 0.0, p;
+        for (int at = 0; (p = above(at)) > 1e-4; at += routes) n += p;
+        return active * n;
+    };
+    const double wide = 1.0 - std::pow(1.0 - above(32), active);  // some expert is above one column
+    const double cus = device_cus(), rows128 = (N + 127LL) / 128 / cus, rows64 = (N + 63LL) / 64 / cus;
+    const double stages = K / kQSuper, quarter = (K / kQSuper + 3) / 4;  // a K-sliced wave's
+    const double cols = tiles(32);
+    const double tiled =
+        3.62 + std::hypot(4.05 + stages * (0.802 + 0.893 * wide),
+                          rows128 * (tiles(128) * (1.803 + 0.2886 * stages) + cols * (0.716 + 0.3647 * stages)));
+    const double one = 4.91 + std::hypot(1.12 + 1.079 * quarter, rows64 * cols * (1.313 + 0.2944 * stages));
+    const double two =
+        5.11 + std::hypot(1.11 + quarter * (1.079 + 0.670 * wide),
+                          rows64 * (tiles(64) * (0.515 + 0.1509 * stages) + cols * (0.887 + 0.1484 * stages)));
+    if (1.03 * std::min(one, two) >= tiled) return 0;
+    return one < two ? 1 : 2;
 }
 
 hipError_t run_grouped(const void *w, const void *w2, int n_split, const void *xq, const int32_t *offsets,
                        int n_experts, const int32_t *route_dst, float *y, int K, int N, int n_routes, bool split,
                        hipStream_t s) {
-    if (const int cols = grouped_kslice_cols(n_routes, n_experts, K); cols > 0)
+    if (const int cols = grouped_kslice_cols(n_routes, n_experts, K, N); cols > 0)
         return launch_gemm_kslice_grouped(w, w2, xq, y, nullptr, K, N, n_routes, n_split, offsets, n_experts,
                                           route_dst, split, cols, s);
     return launch_gemm_mfma_grouped(w, xq, offsets, n_experts, route_dst, y, K, N, n_routes, s, w2, n_split, split);
@@ -634,7 +667,7 @@ hipError_t run_grouped(const void *w, const void *w2, int n_split, const void *x
 
 hipError_t run_gate_up_swiglu(const void *w_gate, const void *w_up, const void *xq, const int32_t *offsets,
                               int n_experts, void *mid_q8_1, int K, int I, int n_routes, bool split, hipStream_t s) {
-    if (const int cols = grouped_kslice_cols(n_routes, n_experts, K); cols > 0)
+    if (const int cols = grouped_kslice_cols(n_routes, n_experts, K, 2 * I); cols > 0)
         return launch_gemm_kslice_grouped(w_gate, w_up, xq, nullptr, mid_q8_1, K, 2 * I, n_routes, I, offsets,
                                           n_experts, nullptr, split, cols, s);
     return launch_gemm_gate_up_swiglu_q8_1(w_gate, w_up, xq, offsets, n_experts, mid_q8_1, K, I, n_routes, s, split);
@@ -683,6 +716,46 @@ int mat_mul_q4_0s_q8_1_grouped_device(const void *d_w_split, const void *d_x_q8_
                                      ncols_k, nrows_out, n_routes, true, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "grouped gemm (split layout) launch");
     return JJO_OK;
+}
+
+int jjo_grouped_auto_kernel(int ncols_k, int nrows_out, int n_routes, int n_experts) {
+    clear_error();
+    const void *a = reinterpret_cast<const void *>(16);
+    if (validate_mm(a, a, a, ncols_k, nrows_out, n_routes) != JJO_OK) return -1;
+    if (n_experts <= 0 || n_experts > 4096) {
+        set_error(JJO_ERR_INVALID_ARG, "1 <= n_experts <= 4096 required");
+        return -1;
+    }
+    if (check_grouped_grid(n_routes, n_experts) != JJO_OK) return -1;
+    if (grouped_gemv(n_routes, ncols_k)) return JJO_ALGO_GEMV;
+    const int cols = grouped_kslice_cols(n_routes, n_experts, ncols_k, nrows_out);
+    return cols > 0 ? JJO_KERNEL_KSLICE + cols : JJO_ALGO_MFMA;
+}
+
+int jjo_grouped_kernel_device(const void *d_w, const void *d_x_q8_1, const int32_t *d_expert_offsets, int n_experts,
+                              const int32_t *d_route_dst, float *d_y, int ncols_k, int nrows_out, int n_routes,
+                              int split, int kernel, void *stream) {
+    clear_error();
+    int rc = split ? validate_split(d_w, d_x_q8_1, d_y, ncols_k, nrows_out, n_routes)
+                   : validate_mm(d_w, d_x_q8_1, d_y, ncols_k, nrows_out, n_routes);
+    if (rc != JJO_OK) return rc;
+    if (d_expert_offsets == nullptr || n_experts <= 0 || n_experts > 4096)
+        return set_error(JJO_ERR_INVALID_ARG, "expert_offsets must be non-null and 1 <= n_experts <= 4096");
+    if ((rc = check_grouped_grid(n_routes, n_experts)) != JJO_OK) return rc;
+    const int cols = kernel - JJO_KERNEL_KSLICE;
+    const bool sliced = (cols == 1 || cols == 2) && ncols_k < kMaxTileK &&
+                        (int64_t)(n_routes + 32 * cols - 1) / (32 * cols) + n_experts <= 65535;
+    if (!sliced && kernel != JJO_ALGO_MFMA)
+        return set_error(JJO_ERR_INVALID_ARG, "kernel %d does not run ncols_k=%d n_routes=%d n_experts=%d", kernel,
+                         ncols_k, n_routes, n_experts);
+    if ((rc = require_gfx950()) != JJO_OK) return rc;
+    const hipError_t e =
+        sliced ? launch_gemm_kslice_grouped(d_w, nullptr, d_x_q8_1, d_y, nullptr, ncols_k, nrows_out, n_routes, 0,
+                                            d_expert_offsets, n_experts, d_route_dst, split != 0, cols,
+                                            (hipStream_t)stream)
+               : launch_gemm_mfma_grouped(d_w, d_x_q8_1, d_expert_offsets, n_experts, d_route_dst, d_y, ncols_k,
+                                          nrows_out, n_routes, (hipStream_t)stream, nullptr, 0, split != 0);
+    return e == hipSuccess ? JJO_OK : hip_fail(e, "grouped gemm launch");
 }
 
 int mat_mul_q4_0_q8_1(const void *weight_q4_0, const float *input, uint8_t *quant_workspace,

@@ -52,7 +52,29 @@ def test_launch_fits_the_grid(K, N, M):
     assert capi.mm_auto_kernel(1536, (1 << 28) - 256, 17) == capi.KERNEL_KSLICE  # the most that fits
 
 
+@pytest.mark.parametrize("K,N,R,E,kernel", [
+    (4096, 256, 48, 8, "gemv"), (14336, 256, 48, 8, "gemv"),
+    (2048, 2816, 800, 64, 1), (1408, 2048, 800, 64, 1),  # 100 tokens, 64 experts top-8: gate|up, down
+    (4096, 28672, 49, 8, 1), (4096, 1024, 48 * 8, 8, 1), (2048, 256, 80 * 8, 8, 1),
+    (4096, 28672, 40 * 8, 8, 2), (14336, 4096, 40 * 8, 8, 2), (2048, 2816, 48 * 64, 64, 2),
+    (4096, 28672, 1024, 8, "tiles"), (14336, 4096, 1024, 8, "tiles"), (4096, 1024, 81 * 8, 8, "tiles"),
+    # tiles that fill the chip, many routes or short rows
+    (2048, 2816, 80 * 64, 64, "tiles"), (128, 14336, 7 * 64, 64, "tiles"), (128, 14336, 80 * 8, 8, "tiles"),
+    (256, 4096, 16 * 64, 64, "tiles"), (256, 4096, 64 * 64, 64, "tiles"), (512, 8192, 64 * 64, 64, "tiles"),
+])
+def test_grouped(K, N, R, E, kernel):
+    want = {"gemv": capi.ALGO_GEMV, "tiles": capi.ALGO_MFMA}.get(kernel)
+    assert capi.grouped_auto_kernel(K, N, R, E) == (capi.KERNEL_KSLICE + kernel if want is None else want)
+
+
 def test_invalid_calls_are_refused():
+    for bad in ((96, 64, 64, 4), (128, 0, 64, 4), (128, 64, 0, 4), (128, 64, 64, 0), (128, 64, 64, 4097)):
+        with pytest.raises(capi.JJOError):
+            capi.grouped_auto_kernel(*bad)
+    i0 = ctypes.c_void_p(16)
+    for kernel in (0, capi.ALGO_GEMV, capi.KERNEL_KSLICE, capi.KERNEL_KSLICE + 3):
+        assert capi.lib().jjo_grouped_kernel_device(i0, i0, i0, 4, None, i0, 128, 64, 64, 0, kernel,
+                                                    None) == capi.JJO_ERR_INVALID_ARG
     with pytest.raises(capi.JJOError):
         capi.mm_auto_kernel(96, 4, 1)
     a16 = ctypes.c_void_p(16)

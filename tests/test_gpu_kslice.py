@@ -100,13 +100,14 @@ def test_kslice_special_scales(dev):
 
 
 @pytest.mark.parametrize("counts,N,K", [
-    # one column tile (mean of at most 24 routes per expert): full, tail, empty and single-route experts
+    # full tiles, tails, empty and single-route experts; with two column tiles, tails that run
+    # the one-column loop
     ([32, 0, 1, 33, 31, 5, 64], 96, 384), ([20] * 3, 65, 128), ([2] * 30 + [70], 257, 1152),
-    # two column tiles, tails that run the one-column loop
     ([64, 65, 1, 0, 96, 97, 32, 33], 130, 640), ([128, 31], 64, 256),
 ])
 def test_kslice_grouped(counts, N, K, dev):
-    """The grouped form at its tile edges, scattered outputs, both layouts (equal bits)."""
+    """The grouped form with one and two column tiles at its tile edges, scattered outputs,
+    both layouts (equal bits in all four), and what the entry chooses for the shape."""
     import torch
     E, R = len(counts), sum(counts)
     assert R > 48  # below, the grouped entry is a GEMV
@@ -125,13 +126,14 @@ def test_kslice_grouped(counts, N, K, dev):
     w = torch.from_numpy(np.concatenate(ws)).to(dev)
     w_split = torch.empty_like(w)
     capi.q4_0_to_split(w, w_split, E * N, K)
+    xq, off, dst = (torch.from_numpy(v).to(dev) for v in (xq, off, dst))
     got = []
     for split in (False, True):
-        y = torch.full((R * N + 64,), float("nan"), dtype=torch.float32, device=dev)
-        capi.grouped_mat_mul(w_split if split else w, torch.from_numpy(xq).to(dev), torch.from_numpy(off).to(dev), y, K,
-                             N, R, route_dst=torch.from_numpy(dst).to(dev), split=split)
-        torch.cuda.synchronize()
-        assert torch.isnan(y[R * N:]).all()
-        got.append(y[:R * N].cpu().numpy().reshape(R, N))
-        np.testing.assert_allclose(got[-1], exp, rtol=RTOL, atol=ATOL)
-    assert np.array_equal(got[0], got[1])
+        wt = w_split if split else w
+        for cols in (1, 2):
+            got.append(_run(lambda y: capi.grouped_kernel(wt, xq, off, y, K, N, R, capi.KERNEL_KSLICE + cols,
+                                                          route_dst=dst, split=split), R, N, dev))
+            np.testing.assert_allclose(got[-1], exp, rtol=RTOL, atol=ATOL)
+        chosen = _run(lambda y: capi.grouped_mat_mul(wt, xq, off, y, K, N, R, route_dst=dst, split=split), R, N, dev)
+        np.testing.assert_allclose(chosen, exp, rtol=RTOL, atol=ATOL)
+    assert all(np.array_equal(got[0], g) for g in got[1:])

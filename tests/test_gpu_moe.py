@@ -121,6 +121,9 @@ MOE_CASES = [  # T, H, I, E, top_k
     (64, 256, 256, 64, 8),     # many experts, top-8: mostly short (narrow / paired) tiles
     (40, 128, 128, 256, 8),    # 256 experts for 320 routes: most get 0..3
     (33, 1024, 384, 8, 2),     # wider hidden size
+    (170, 256, 384, 4, 2),     # a mean of 85 routes: the 128-route tiles
+    (131, 256, 1664, 6, 2),    # gate|up in two column tiles per workgroup
+    (256, 768, 384, 24, 4),    # the same, and the down projection
 ]
 # Decode-sized batches: the FFN runs its expert matrices as routed GEMVs (a
 # token's experts are distinct, so no expert holds more than T routes).
@@ -143,7 +146,7 @@ MOE_DECODE_CASES = [  # T, H, I, E, top_k
     (2, 512, 5120, 4, 2),      # down projection K = 5120: two K slices
     (1, 9216, 256, 4, 2),      # gate|up K = 9216: three K slices
     (3, 16384, 128, 3, 1),     # gate|up K = 16384: four K slices
-    (16, 128, 128, 32, 25),    # 400 routes: routing in four launches, then the routed GEMVs
+    (16, 128, 128, 32, 25),    # 400 routes: routing in two launches, then the routed GEMVs
 ]
 
 
@@ -540,9 +543,9 @@ def _split_stack(w_dev, rows, K, dev):
                                         ([0] * 200 + [3] + [0] * 50 + [7, 1] + [0] * 11, 64, 512)])
 def test_grouped_split_layout(counts, N, K, dev):
     """The grouped GEMM on split-layout experts equals the block_q4_0 launch bit for
-    bit above 48 routes (the same MFMA kernel; only the weight loads differ), with route
-    scatter, empty experts, narrow and paired tails and a ragged N.  At 48 routes or
-    fewer both run as routed GEMVs, whose two layouts sum a row in different orders:
+    bit above 48 routes (the same MFMA kernel, the chosen one and the 128-route tiles by
+    name; only the weight loads differ), with route scatter, empty experts, narrow and
+    paired tails and a ragged N.  At 48 routes or fewer both run as routed GEMVs, whose two layouts sum a row in different orders:
     both are checked against the oracle, scattered through route_dst."""
     import torch
     E = len(counts)
@@ -565,6 +568,12 @@ def test_grouped_split_layout(counts, N, K, dev):
     assert not np.isnan(a).any()
     if R > GROUPED_GEMV_ROUTES:
         assert np.array_equal(a, b)
+        for v, y, split in ((w, y1, False), (ws, y2, True)):
+            y.fill_(float("nan"))
+            capi.grouped_kernel(v, xq_d, off_d, y, K, N, R, capi.ALGO_MFMA, route_dst=dst, split=split)
+        tiles = host(y1)
+        assert np.array_equal(tiles, host(y2))
+        np.testing.assert_allclose(tiles, a, rtol=RTOL, atol=ATOL)
     else:
         ref = np.zeros((R, N), dtype=np.float32)
         blocks = xq.reshape(K // 128, R, 144)

@@ -388,8 +388,9 @@ def test_grouped_moe_small(dev):
 
 @pytest.mark.parametrize("counts", [[1, 129, 0, 31, 160, 32, 33, 7], [3, 2, 1, 4], [64, 65, 0, 96, 1, 200],
                                     [8, 9, 136, 137, 5, 6], [161, 320, 321, 481, 0, 2]])
-def test_grouped_tail_tiles(counts, dev):
-    """Experts of 1..33 routes (one narrow chunk of 1..2 column tiles), 129..160 (one
+@pytest.mark.parametrize("kernel", [0, capi.ALGO_MFMA])
+def test_grouped_tail_tiles(counts, kernel, dev):
+    """What the entry chooses, and the 128-route tiles by name.  Experts of 1..33 routes (one narrow chunk of 1..2 column tiles), 129..160 (one
     chunk of up to 5 column tiles), 161..481 (2..4 equal chunks, the last ones
     ragged), and empty experts; every output row is checked against the oracle."""
     import torch
@@ -402,8 +403,11 @@ def test_grouped_tail_tiles(counts, dev):
     ws = [make_w(N, K, 60 + e) for e in range(E)]
     dst = np.random.default_rng(1).permutation(R).astype(np.int32)
     y = torch.full((R * N,), float("nan"), dtype=torch.float32, device=dev)
-    capi.grouped_mat_mul(to_dev(np.concatenate(ws), dev), to_dev(xq, dev), to_dev(offsets, dev), y, K, N, R,
-                         route_dst=to_dev(dst, dev))
+    args = (to_dev(np.concatenate(ws), dev), to_dev(xq, dev), to_dev(offsets, dev), y, K, N, R)
+    if kernel:
+        capi.grouped_kernel(*args, kernel, route_dst=to_dev(dst, dev))
+    else:
+        capi.grouped_mat_mul(*args, route_dst=to_dev(dst, dev))
     torch.cuda.synchronize()
     got = y.cpu().numpy().reshape(R, N)
     assert not np.isnan(got).any()
