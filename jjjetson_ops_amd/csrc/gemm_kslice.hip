@@ -104,8 +104,8 @@ __device__ __forceinline__ void kslice_loop(f32x16 (&acc)[RT][CT], uint8_t *stag
     // Inline asm: the compiler would order every later LDS access behind these; their
     // completion is waited for at the top of a stage.
     constexpr int kPieces = 3 * RT + L::kXRuns;
-    // One DMA instruction of a stage, for the spread form: the weights, which come from
-    // further away, first.
+    // One DMA instruction of a stage.  The spread form takes them in this order: the weights,
+    // which come from further away, first.
     auto dma_piece = [&](int k, int s) {
         if (k >= 3 * RT) {
             const int i = k - 3 * RT;
@@ -136,40 +136,10 @@ __device__ __forceinline__ void kslice_loop(f32x16 (&acc)[RT][CT], uint8_t *stag
                          : "v"(woff[rt][i]), "s"(wd[rt] + (size_t)s * 8), "{m0}"(m0v)
                          : "memory");
     };
+    // A whole stage in one burst: the activations, then the weights.
     auto dma = [&](int s) {
-        const uint8_t *px = xb + (size_t)s * x_stride;
 #pragma unroll
-        for (int i = 0; i < L::kXRuns; ++i) {
-            const uint32_t m0v = __builtin_amdgcn_readfirstlane(stage_lds + i * 1024);
-            if ((i + 1) * 1024 <= L::kXBytes || lane < 32)
-                asm volatile("global_load_lds_dwordx4 %0, %1"
-                             :
-                             : "v"(min((uint32_t)(i * 1024 + lane * 16), xlim)), "s"(px), "{m0}"(m0v)
-                             : "memory");
-        }
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) {
-            const uint32_t dst = stage_lds + L::kOffW + rt * L::kWTile;
-#pragma unroll
-            for (int i = 0; i < 3; ++i) {
-                const uint32_t m0v = __builtin_amdgcn_readfirstlane(dst + i * 1024);
-                if constexpr (!SPLIT)
-                    asm volatile("global_load_lds_dwordx3 %0, %1"
-                                 :
-                                 : "v"(woff[rt][i]), "s"(wq[rt] + (size_t)s * (4 * kQ4BlockBytes)), "{m0}"(m0v)
-                                 : "memory");
-                else if (i < 2)
-                    asm volatile("global_load_lds_dwordx4 %0, %1"
-                                 :
-                                 : "v"(woff[rt][i]), "s"(wq[rt] + (size_t)s * 64), "{m0}"(m0v)
-                                 : "memory");
-                else
-                    asm volatile("global_load_lds_dword %0, %1"
-                                 :
-                                 : "v"(woff[rt][i]), "s"(wd[rt] + (size_t)s * 8), "{m0}"(m0v)
-                                 : "memory");
-            }
-        }
+        for (int k = 0; k < kPieces; ++k) dma_piece((k + 3 * RT) % kPieces, s);
     };
 
     i32x16 bias;
