@@ -1188,7 +1188,8 @@ int moe_ffn_run(bool split, void *stream, const float *x, const float *logits, c
     hipError_t e;
     if (moe_decode_path(T, H, I, E, top_k)) {
         // Chunk size of the routed GEMVs: the mean routes per active expert (an expert
-        // with more takes several chunks with its weights held in registers).
+        // with more takes several chunks; at a mean of one a route is a workgroup of its
+        // own, and an expert's later routes read its rows through L2).
         // 1) quantize + top-k + dispatch + gather, 2) gate|up (both matrices, one
         // launch) -> fp32 [R][2I], 3) SwiGLU + Q8_1, 4) down projection, 5) combine
         if (R <= kMoeDecodeRoutes) {

@@ -27,10 +27,14 @@
 //   * One buffer per wave, not a ring: deeper rings hid no more latency and cost
 //     residency (64 x 64 tiles, 256 tokens, N=14336, block_q4_0: 83 us with two weight
 //     slots, 59 with one).
-//   * The loop is bound by instruction issue: a wave issues a two-operand VALU
-//     instruction every 5.0 clocks and a three-operand one every 6.1, a SIMD every 2.5
-//     and 3.1 from two waves on, and MFMA time adds to it almost in full.  So what is
-//     minimised is instructions per 32x32 block: weights are expanded with one load of
+//   * The 64 x 64 forms' loop is bound by instruction issue: a wave issues a two-operand
+//     VALU instruction every 5.0 clocks and a three-operand one every 6.1, a SIMD every 2.5
+//     and 3.1 from two waves on, and MFMA time adds to it almost in full (K=11008,
+//     N=4096, 777 tokens: 651 VALU instructions per wave and stage, 512 of them the epilogue;
+//     waves are ready but not issued for 21% of their cycles and wait for 16%; MFMA busy 18%;
+//     the two rounds of workgroups are 81% full).  The 32 x 32 form waits: K=11008, N=4096,
+//     24 tokens is 128 workgroups, half the CUs, whose waves wait for 67% of their cycles.
+//     What is minimised is instructions per 32x32 block: weights are expanded with one load of
 //     two blocks per lane pair and v_permlane32_swap (no duplicated work in the two lane
 //     halves), scales are widened to fp32 once per stage, d_x stays an fp32 register (a
 //     v_fma_mix would issue at two thirds of the rate), and the next block's MFMA is
@@ -476,9 +480,9 @@ hipError_t launch_gemm_kslice(const void *w, const void *xq, float *y, int K, in
 hipError_t launch_gemm_kslice_grouped(const void *w, const void *w2, const void *xq, float *y, void *midq, int K,
                                       int N, int M, int n_split, const int32_t *offsets, int n_experts,
                                       const int32_t *route_dst, bool split, int cols, hipStream_t stream) {
-    // Four waves: two (64 routes) or three (32 routes) workgroups share a CU, and an
-    // expert's ragged last tile ends sooner than with eight (E=64 top-8, 100 tokens, FFN:
-    // 137 us against 195).
+    // Four waves: two workgroups share a CU, three at 32 routes with SwiGLU (167 registers;
+    // 170 without), and an expert's ragged last tile ends sooner than with eight (E=64
+    // top-8, 100 tokens, FFN: 137 us against 195).
     auto go = [&](auto ct, auto sp, auto sw) {
         return launch_grouped<decltype(ct)::value, 4, decltype(sp)::value, decltype(sw)::value>(
             w, w2, xq, y, midq, K, N, M, n_split, offsets, n_experts, route_dst, stream);

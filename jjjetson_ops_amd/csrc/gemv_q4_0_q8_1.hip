@@ -289,13 +289,15 @@ __device__ __forceinline__ void finish_f32(uint8_t *xs, uint8_t *__restrict__ xq
 // selects the slot-th expert that has routes (which = 1: the second stacked
 // matrix w2, written N columns further along each output row).  The workgroup
 // keeps its weight rows in registers and takes the expert's routes M at a time
-// (each chunk re-stages only activation rows), so every weight byte of an active
+// (each chunk re-stages only activation rows), so at M > 1 every weight byte of an active
 // expert is read once whatever its route count.  Output row p (a sorted route
 // position) starts at y + p * ldy, or at y + route_dst[p] * ldy.
 // M = 1 (a mean of at most one route per active expert): a slot is one route instead,
 // and the workgroups that read the same rows for an expert's routes are 8 apart in the
 // grid (blockIdx.x = 8 * slot + row group % 8, blockIdx.y = row group / 8, blockIdx.z =
-// which): the same XCD at the same time, so the later ones read its L2.  A second pass
+// which): the same XCD at the same time, so the later ones read its L2 (four tokens on six
+// of eight experts, two of them with two routes: 1.10 times the weights fetched from HBM
+// by gate|up, 1.06 by down; one route each 1.00).  A second pass
 // of one workgroup re-read the rows after they had left the cache and lengthened the
 // grid's tail: E=8 top-2 4096 x 14336, random routing, FFN us (block_q4_0 / split), T=2
 // 67.0 / 69.7 -> 49.1 / 55.8, T=4 125.1 / 124.3 -> 108.6 / 103.4; one route on every expert
