@@ -994,7 +994,7 @@ int check_moe_shape(int num_tokens, int hidden, int inter, int num_experts, int 
 struct MoeWs {
     float *route_w;
     int32_t *ids, *offsets, *src_route, *dst_of_route;
-    uint8_t *xq, *xp, *midq;
+    uint8_t *xp, *midq;
     float *eout;
     float *gate_up;  // [R][2I] fp32, decode path only
     int64_t bytes;
@@ -1019,7 +1019,9 @@ bool moe_decode_path(int T, int H, int I, int E, int top_k) {
     return (T <= JJO_MOE_GEMV_TOKENS || sparse) && H <= 16384 && I <= 16384;
 }
 
-// Workspace carve-up, every part 256-byte aligned.
+// Workspace carve-up, every part 256-byte aligned.  No launch uses the T Q8_1 rows before xp any
+// more (the routing quantizes straight into xp); they stay reserved, so that the parts after
+// them and the workspace's size are where callers that read the tables expect them.
 MoeWs moe_ws_layout(uint8_t *base, int T, int H, int I, int E, int top_k) {
     const int64_t R = (int64_t)T * top_k;
     int64_t off = 0;
@@ -1034,7 +1036,7 @@ MoeWs moe_ws_layout(uint8_t *base, int T, int H, int I, int E, int top_k) {
     w.offsets = (int32_t *)take((int64_t)(E + 1) * 4);
     w.src_route = (int32_t *)take(R * 4);
     w.dst_of_route = (int32_t *)take(R * 4);
-    w.xq = take((int64_t)T * (H / kQSuper) * kQ8BlockBytes);
+    (void)take((int64_t)T * (H / kQSuper) * kQ8BlockBytes);
     w.xp = take(R * (H / kQSuper) * kQ8BlockBytes);
     w.midq = take(R * (I / kQSuper) * kQ8BlockBytes);
     w.eout = (float *)take(R * H * 4);
